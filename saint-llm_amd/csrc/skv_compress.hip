@@ -13,6 +13,8 @@
 // state of each channel (max, sum, weighted sum; fp32 [batch, 3, channels]),
 // so a decode step costs O(channels) whatever m is, and a block emits from
 // that state the same value a one-shot pooling of its m tokens gives.
+#include <algorithm>
+
 #include "skv_pool_state.h"
 
 namespace skv {
@@ -38,84 +40,251 @@ struct CompressArgs {
   int channels;
   int format;
   int fp8_main;  // main (quantized) channels in FP8 format
-  int in_f32;    // c/z rows are fp32
 };
 
-__device__ __forceinline__ void state_emit(const PoolState& st, const CompressArgs& a, int b, int64_t e,
-                                           int lane, int groups) {
-  const int64_t page_idx = e / a.bs;
-  const int32_t page = (page_idx < a.bt_stride) ? a.bt[b * a.bt_stride + page_idx] : -1;
-  if (page < 0 || page >= a.n_pages) return;  // wave-uniform
-  uint8_t* entry = a.pool + (static_cast<int64_t>(page) * a.bs + e % a.bs) * a.entry_bytes;
-  state_emit_entry(st, entry, lane, groups, a.format, a.fp8_main);
-}
+// Work split.  The pooling is independent per channel, so a workgroup takes a
+// block of 128 channels (one fp8 scale block): 16 lanes of 8 channels read
+// 256 consecutive bytes of a token row, and the 16 lane groups of its 4 waves
+// are shared out between entries and token slices.  kSlices lane groups fold
+// the tokens of one entry in turn, 4 tokens of a lane in flight at once, and
+// are merged by lane shuffles (and through LDS for 16 slices); the other lane
+// groups hold other entries.  A block of 4 tokens needs no slices (16 entries
+// per workgroup); one of 128 takes all 16 lane groups, 8 tokens each.
+// HBM-bound: c and z rows are read once.  One wave folding an entry's tokens one
+// after another, with a memory round trip each, took 1.45 us per token.  4
+// sequences of 6,700-8,192 tokens x 576 bf16 channels: entries of 4 tokens 25.4 us
+// (3.0 TB/s; the call averaged 247 us before), of 128 tokens 26 us; 16 x 8,192
+// tokens 86 us (3.95 TB/s, a plain copy 4.9); two sequences of 95 and 300 tokens 5.5
+// and, with blocks of 128, 8.3 us (186 before).
+constexpr int kCmThreads = 256;
+constexpr int kCmWaves = kCmThreads / kWave;
+constexpr int kCmLanes = 16;                         // lanes per 128-channel token row
+constexpr int kCmGroups = kCmThreads / kCmLanes;     // lane groups per workgroup
+constexpr int kCmFold = 4;                           // tokens in flight per lane
 
-// Token rows [p0, p1) of sequence b (all new in this call) folded into st.
-__device__ __forceinline__ void fold_tokens(PoolState& st, const CompressArgs& a, int b, int64_t first_new,
-                                            int64_t p0, int64_t p1, int lane, int groups) {
-  for (int64_t p = p0; p < p1; ++p) {
-    const int64_t i = p - first_new;
-    const uint8_t* crow = a.c_new + b * a.in_seq_stride + i * a.in_row_stride;
-    const uint8_t* zrow = a.z_new + b * a.in_seq_stride + i * a.in_row_stride;
-    const float* brow = a.bias + (p % a.m) * a.channels;
-    if (a.in_f32) {  // uniform: fp32 rows
-      state_update(st, reinterpret_cast<const float*>(crow), reinterpret_cast<const float*>(zrow), brow, lane,
-                   groups);
+struct CompressSmem {
+  float mx[kCmWaves][8][kCmLanes];  // of 16 slices: each wave's max, then its sums from the common max
+  float sum[kCmWaves - 1][8][kCmLanes], acc[kCmWaves - 1][8][kCmLanes];
+};
+
+// A lane's 8 channels of a row as they lie in memory (bf16 or fp32).
+template <class Row>
+struct RawRow {
+  static constexpr int kVecs = sizeof(Row) / 2;  // 16-byte pieces
+  u32x4 v[kVecs];
+  __device__ __forceinline__ void load(const uint8_t* row, int grp) {
+    const u32x4* p = reinterpret_cast<const u32x4*>(row + grp * 16 * kVecs);
+#pragma unroll
+    for (int i = 0; i < kVecs; ++i) v[i] = p[i];
+  }
+  __device__ __forceinline__ void get(float* f) const {
+    if constexpr (kVecs == 1) {
+      unpack8_bf16(v[0], f);
     } else {
-      state_update(st, reinterpret_cast<const uint16_t*>(crow), reinterpret_cast<const uint16_t*>(zrow), brow,
-                   lane, groups);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) f[j] = __uint_as_float(v[j >> 2][j & 3]);
     }
   }
-}
-
-// grid: (units, batch); block: one wave.
-//   unit 0      : block e0 (continuing from the stored state when the previous
-//                 call left it incomplete); then, if further blocks complete and
-//                 the last one stays incomplete, the state of that last block.
-//   unit k >= 1 : complete block e0 + k (only new tokens).
-// Only unit 0 touches the state buffer of its sequence.
-__global__ __launch_bounds__(kPoolWave) void k_compress_append(CompressArgs a) {
-  const int b = blockIdx.y;
-  const int k = blockIdx.x;
-  const int lane = threadIdx.x;
-  const int64_t L = a.lens[b];
-  const int64_t n = a.n_new ? a.n_new[b] : a.n_uni;
-  if (n <= 0 || n > L || n > a.in_len) return;
-  const int64_t first_new = L - n;
-  const int64_t e0 = first_new / a.m;
-  const int64_t e1 = L / a.m;  // entries [e0, e1) complete in this call
-  const int64_t nb = e1 - e0;
-  if (k >= max<int64_t>(nb, 1)) return;
-  const int groups = a.channels >> 3;
-  float* sbase = a.state + static_cast<int64_t>(b) * 3 * a.channels;
-  PoolState st;
-  if (k == 0) {
-    if (first_new % a.m != 0) {
-      state_load(st, sbase, a.channels, lane, groups);
-    } else {
-      state_reset(st);
+  // every channel `bits` (the bits of a value of this type) where dead
+  __device__ __forceinline__ void fill(bool dead, uint32_t bits) {
+    const uint32_t word = kVecs == 1 ? bits | (bits << 16) : bits;
+#pragma unroll
+    for (int i = 0; i < kVecs; ++i) {
+#pragma unroll
+      for (int q = 0; q < 4; ++q) v[i][q] = dead ? word : v[i][q];
     }
-    const int64_t p1 = min(L, (e0 + 1) * a.m);
-    fold_tokens(st, a, b, first_new, first_new, p1, lane, groups);
-    if (p1 == (e0 + 1) * a.m) {
-      state_emit(st, a, b, e0, lane, groups);
-      if (nb >= 1 && L % a.m != 0) {
-        // the incomplete last block e1 starts fresh; its state replaces the
-        // one loaded above (same lanes, after the loads retired)
-        __syncthreads();
-        state_reset(st);
-        fold_tokens(st, a, b, first_new, e1 * a.m, L, lane, groups);
-        state_store(st, sbase, a.channels, lane, groups);
+  }
+};
+
+// Tokens first + slice + stride * i < p1 of entry e (sequence b) folded into
+// st.  Every load of a turn is issued before any is used (left to itself the
+// compiler waits for each row in turn: 14.8 us for a call of a few entries).
+template <class Row>
+__device__ __forceinline__ void fold_tokens(PoolLane& st, const CompressArgs& a, int b, int first_new, int e, int first,
+                                            int p1, int slice, int stride, int grp) {
+  typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // bias is 4-byte aligned
+  const uint8_t* cbase = a.c_new + b * a.in_seq_stride;
+  const uint8_t* zbase = a.z_new + b * a.in_seq_stride;
+  for (int p = first + slice; p < p1; p += kCmFold * stride) {
+    RawRow<Row> cr[kCmFold], zr[kCmFold];
+    f32x4u br[kCmFold][2];
+    bool live[kCmFold];
+#pragma unroll
+    for (int u = 0; u < kCmFold; ++u) {
+      const int pu = p + u * stride;
+      live[u] = pu < p1;
+      const int q = live[u] ? pu : p;  // a row that exists
+      const int64_t off = (q - first_new) * a.in_row_stride;
+      zr[u].load(zbase + off, grp);
+      cr[u].load(cbase + off, grp);
+      const f32x4u* bp = reinterpret_cast<const f32x4u*>(a.bias + static_cast<int64_t>(q - e * a.m) * a.channels + grp * 8);
+      br[u][0] = bp[0];
+      br[u][1] = bp[1];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (__ballot(!live[kCmFold - 1])) {  // tokens past the end: value -inf, row 0
+#pragma unroll
+      for (int u = 1; u < kCmFold; ++u) {
+        zr[u].fill(!live[u], sizeof(Row) == 2 ? 0xff80u : 0xff800000u);
+        cr[u].fill(!live[u], 0u);
       }
-    } else {
-      state_store(st, sbase, a.channels, lane, groups);
     }
-    return;
+    float v[kCmFold][8], c[kCmFold][8];
+#pragma unroll
+    for (int u = 0; u < kCmFold; ++u) {
+      zr[u].get(v[u]);
+      cr[u].get(c[u]);
+#pragma unroll
+      for (int j = 0; j < 8; ++j) v[u][j] += br[u][j >> 2][j & 3];
+    }
+    pool_fold<kCmFold>(st, v, c);
   }
-  const int64_t e = e0 + k;
-  state_reset(st);
-  fold_tokens(st, a, b, first_new, e * a.m, (e + 1) * a.m, lane, groups);
-  state_emit(st, a, b, e, lane, groups);
+}
+
+// The states of the lane groups of one entry, merged: every lane group holds
+// the result for 1 and 4 slices (one lane group, one wave), wave 0 for 16.
+// For 16 slices every thread of the workgroup must call it.
+template <int kSlices>
+__device__ __forceinline__ void merge_slices(CompressSmem& sm, PoolLane& st) {
+  static_assert(kSlices == 1 || kSlices == 4 || kSlices == 16, "one lane group, one wave or the workgroup");
+  if constexpr (kSlices == 1) return;
+  float M[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    M[j] = __builtin_elementwise_maximum(st.mx[j], __shfl_xor(st.mx[j], 16));
+    M[j] = __builtin_elementwise_maximum(M[j], __shfl_xor(M[j], 32));
+  }
+  pool_rebase(st, M);
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    st.sum[j] += __shfl_xor(st.sum[j], 16);
+    st.acc[j] += __shfl_xor(st.acc[j], 16);
+    st.sum[j] += __shfl_xor(st.sum[j], 32);
+    st.acc[j] += __shfl_xor(st.acc[j], 32);
+  }
+  if constexpr (kSlices == 16) {
+    const int wave = threadIdx.x / kWave, l = threadIdx.x % kCmLanes;
+    if (threadIdx.x % kWave < kCmLanes) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) sm.mx[wave][j][l] = st.mx[j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < 8; ++j) {
+      M[j] = sm.mx[0][j][l];
+#pragma unroll
+      for (int w = 1; w < kCmWaves; ++w) M[j] = __builtin_elementwise_maximum(M[j], sm.mx[w][j][l]);
+    }
+    pool_rebase(st, M);
+    if (wave > 0 && threadIdx.x % kWave < kCmLanes) {
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        sm.sum[wave - 1][j][l] = st.sum[j];
+        sm.acc[wave - 1][j][l] = st.acc[j];
+      }
+    }
+    __syncthreads();
+    if (wave == 0) {
+#pragma unroll
+      for (int w = 0; w < kCmWaves - 1; ++w) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          st.sum[j] += sm.sum[w][j][l];
+          st.acc[j] += sm.acc[w][j][l];
+        }
+      }
+    }
+  }
+}
+
+// The block-table slot of entry e of sequence b (the caller reads it ahead of
+// the fold, with the first round trip).
+__device__ __forceinline__ int32_t entry_page(const CompressArgs& a, int b, int e) {
+  return a.bt[b * a.bt_stride + min<int64_t>(e / a.bs, a.bt_stride - 1)];
+}
+
+// Entry e, in page `page` of its table, from its channels' states (16 lanes, 8 channels each).
+__device__ __forceinline__ void emit_entry(const PoolLane& st, const CompressArgs& a, int e, int32_t page, int grp,
+                                           int groups) {
+  const int page_idx = e / a.bs;
+  if (page_idx >= a.bt_stride || page < 0 || page >= a.n_pages) return;  // uniform over the lane group
+  uint8_t* entry = a.pool + (static_cast<int64_t>(page) * a.bs + (e - page_idx * a.bs)) * a.entry_bytes;
+  float out[8];
+#pragma unroll
+  for (int j = 0; j < 8; ++j) out[j] = grp < groups ? pool_out(st, j) : 0.f;
+  if (a.format != SKV_FMT_F32) {
+#pragma unroll
+    for (int j = 0; j < 8; j += 2) bf16_round2(out[j], out[j + 1]);  // a bf16 compressor's entries
+  }
+  store_entry_group(entry, out, grp, groups, a.format, a.fp8_main);
+}
+
+// grid: (workgroups over the blocks, batch, 128-channel blocks).  Blocks
+// [e0, e1) of a sequence complete in this call; block e0 continues from the
+// stored state when the call before left it incomplete, and the tokens of
+// block e1, when it stays incomplete, go to the state.  When one call does
+// both for different blocks, workgroup 0 takes block e1 in a turn of its own
+// after block e0 (which is its first), so that the state is read before it
+// is written.
+template <class Row, int kSlices>
+__global__ __launch_bounds__(kCmThreads, sizeof(Row) == 2 ? 3 : 2) void k_compress_append(CompressArgs a) {
+  __shared__ CompressSmem sm;
+  constexpr int kEntries = kCmGroups / kSlices;  // per workgroup and turn
+  const int b = blockIdx.y;
+  const int L = a.lens[b];
+  const int n = a.n_new ? a.n_new[b] : a.n_uni;
+  if (n <= 0 || n > L || n > a.in_len) return;
+  const int first_new = L - n;
+  const int e0 = first_new / a.m;
+  const int e1 = L / a.m;
+  const bool resumes = first_new > e0 * a.m;  // block e0 has a stored state
+  const bool leaves = L > e1 * a.m;           // block e1 leaves one
+  bool last_turn = blockIdx.x == 0 && resumes && leaves && e1 > e0;
+  const int n_units = e1 - e0 + (leaves && !(resumes && e1 > e0) ? 1 : 0);
+  const int groups = a.channels >> 3;
+  const int grp = blockIdx.z * kCmLanes + threadIdx.x % kCmLanes;
+  const int gsafe = min(grp, groups - 1);  // lanes past the channels read the last group and store nothing
+  const int slot = threadIdx.x / kCmLanes / kSlices, slice = threadIdx.x / kCmLanes % kSlices;
+  float* sbase = a.state + static_cast<int64_t>(b) * 3 * a.channels + gsafe * 8;
+  int unit0 = blockIdx.x * kEntries;
+  while (unit0 < n_units || last_turn) {
+    const bool in_last = unit0 >= n_units;
+    if (in_last) __syncthreads();  // block e0's lanes have read the state
+    const int unit = in_last ? e1 - e0 + slot : unit0 + slot;
+    const int e = e0 + unit;
+    const bool active = in_last ? slot == 0 : unit < n_units;
+    PoolLane st;
+    pool_reset(st);
+    int32_t page = -1;
+    if (active) {
+      page = entry_page(a, b, e);
+      if (e == e0 && slice == 0 && resumes) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          st.mx[j] = sbase[j];
+          st.sum[j] = sbase[a.channels + j];
+          st.acc[j] = sbase[2 * a.channels + j];
+        }
+      }
+      fold_tokens<Row>(st, a, b, first_new, e, max(first_new, e * a.m), min(L, (e + 1) * a.m), slice, kSlices, gsafe);
+    }
+    merge_slices<kSlices>(sm, st);
+    if (active && slice == 0) {
+      if (e < e1) {
+        emit_entry(st, a, e, page, grp, groups);
+      } else if (grp < groups) {
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          sbase[j] = st.mx[j];
+          sbase[a.channels + j] = st.sum[j];
+          sbase[2 * a.channels + j] = st.acc[j];
+        }
+      }
+    }
+    if (in_last) break;
+    unit0 += gridDim.x * kEntries;
+    if constexpr (kSlices == 16) __syncthreads();  // the LDS is written again
+  }
 }
 
 }  // namespace skv
@@ -178,11 +347,22 @@ extern "C" int skv_compress_append(void* pool, int64_t entry_bytes, int64_t bloc
   a.channels = static_cast<int>(channels);
   a.format = format;
   a.fp8_main = fp8_main;
-  a.in_f32 = in_f32 ? 1 : 0;
-  // at most floor((in_len + m - 1) / m) + 1 blocks complete in one call
-  const int64_t units = (in_len + m - 1) / m + 1;
-  if (units > INT32_MAX) return set_error(SKV_EINVAL, "%s: in_len too large", what);
-  hipLaunchKernelGGL(k_compress_append, dim3(static_cast<unsigned>(units), static_cast<unsigned>(batch)),
-                     dim3(kPoolWave), 0, static_cast<hipStream_t>(stream), a);
+  // slices of an entry: at least 4 tokens per lane, which a turn of fold_tokens takes at once
+  // (blocks of 8 over 4 slices: 54 us for 4 x 8192 tokens of 576 channels, over one: 24 us)
+  const int slices = m < 16 ? 1 : m < 64 ? 4 : 16;
+  // a call's tokens lie in at most ceil(in_len / m) + 1 blocks; past 2^20 workgroups each takes several turns
+  const int64_t turns = ceil_div(ceil_div(in_len, m) + 1, kCmGroups / slices);
+  const dim3 grid(static_cast<unsigned>(std::min<int64_t>(turns, 1 << 20)), static_cast<unsigned>(batch),
+                  static_cast<unsigned>(ceil_div(channels, 8 * kCmLanes)));
+  const auto launch = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, grid, dim3(kCmThreads), 0, static_cast<hipStream_t>(stream), a);
+  };
+  if (in_f32) {
+    slices == 1 ? launch(k_compress_append<float, 1>)
+                : slices == 4 ? launch(k_compress_append<float, 4>) : launch(k_compress_append<float, 16>);
+  } else {
+    slices == 1 ? launch(k_compress_append<uint16_t, 1>)
+                : slices == 4 ? launch(k_compress_append<uint16_t, 4>) : launch(k_compress_append<uint16_t, 16>);
+  }
   return check_launch(what);
 }
