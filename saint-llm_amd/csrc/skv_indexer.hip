@@ -9,6 +9,8 @@
 // path takes no visual bias (csa.py:396-399) and neither does this kernel.
 //
 // The tile (MFMA mapping, operand staging) is in skv_indexer_tile.h.
+#include <algorithm>
+
 #include "skv_common.h"
 #include "skv_indexer_tile.h"
 
@@ -45,6 +47,201 @@ __global__ __launch_bounds__(kIdxThreads, 2) void k_indexer_scores(IndexerArgs a
       sm, r, static_cast<int>(blockIdx.x),
       [&] { return min(a.n_entries[b], a.max_entries); },  // the grid covers max_entries
       [&](int e, float v) { out[e] = v; });
+}
+
+// ---------------------------------------------------------------------------
+// Several query tokens per sequence (a prompt chunk).  The product is a GEMM of
+// the tokens' heads against the sequence's keys, bound by the matrix cores once
+// the keys are shared: a workgroup takes kIrTokens tokens and a run of entries,
+// kIrTile at a time through LDS, and each of its 8 waves keeps one token's query
+// (64 heads x 128 channels) as A operands in registers, so an LDS read of a key
+// operand feeds 4 products.  (k_indexer_scores reads the query from LDS for
+// every 16 entries, one read per product: LDS-bound at 0.43 PFLOP/s.)  Products
+// and head sums run in k_indexer_scores's order: the scores are the same bits.
+// 2,048 tokens x 4,096 entries of 64 heads x 128: 156 us, 0.88 PFLOP/s (323 us
+// before; a large bf16 product of the library runs at 1.27).  Two tokens per
+// wave would halve the key reads but spill.
+// ---------------------------------------------------------------------------
+constexpr int kIrMinTokens = 6;  // fewer query tokens per sequence: k_indexer_scores (see the launch)
+constexpr int kIrThreads = 512;
+constexpr int kIrTokens = kIrThreads / kWave;  // query tokens per workgroup, one per wave
+constexpr int kIrTile = 128;                   // entries per LDS tile
+
+struct IndexerRowsArgs {
+  IndexerArgs a;
+  int32_t groups;  // token groups per sequence
+  int32_t run;     // entries per workgroup, a multiple of kIrTile
+};
+
+// What heads and channels past the query's, and entries without a page, read:
+// no select follows a load.
+__device__ __align__(16) uint8_t g_idx_zero[16];
+
+// HB: 16-head blocks, KS: 32-channel steps (heads and channels past the
+// query's are zero in both operands).
+template <int HB, int KS>
+__global__ __launch_bounds__(kIrThreads, 2) void k_indexer_scores_rows(IndexerRowsArgs ra) {
+  const IndexerArgs& a = ra.a;
+  constexpr int kRow = 32 * KS + 8;  // LDS row of a key (16 bytes of pad: distinct banks)
+  constexpr int kChunks = 4 * KS;    // 16-byte pieces of a key
+  constexpr int kPer = kIrTile * kChunks / kIrThreads;
+  __shared__ alignas(16) uint16_t keys[2][kIrTile][kRow];
+  __shared__ int64_t src_row[3][kIrTile];  // byte offset of each entry's key in the pool, -1 unmapped or past the run;
+                                           // tile i of the run in row i % 3
+  const int tid = threadIdx.x, lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid) / kWave;
+  const int col = lane & 15, grp = lane >> 4;
+  const int b = blockIdx.y / ra.groups;
+  const int t = (blockIdx.y - b * ra.groups) * kIrTokens + wave;  // this wave's token
+  const int n_ent = min(a.n_entries[b], a.max_entries);
+  const int e_lo = blockIdx.x * ra.run, e_hi = min(n_ent, e_lo + ra.run);
+  if (e_lo >= e_hi) return;  // uniform
+  const int32_t* bt_row = a.block_table + static_cast<int64_t>(b) * a.bt_stride;
+  // entry e's page (loaded a tile ahead of its key) and its key's offset
+  const auto page_of = [&](int e) { return bt_row[min(static_cast<int>(udiv24(e, a.block_size)), a.bt_stride - 1)]; };
+  const auto row_of = [&](int e, int32_t page) -> int64_t {
+    const int pi = static_cast<int>(udiv24(e, a.block_size));
+    const bool ok = e < e_hi && pi < a.bt_stride && page >= 0 && page < a.n_pages;
+    return ok ? (static_cast<int64_t>(page) * a.block_size + (e - pi * a.block_size)) * a.c * 2 : -1;
+  };
+  if (tid < 2 * kIrTile) src_row[tid / kIrTile][tid % kIrTile] = row_of(e_lo + tid, page_of(e_lo + tid));
+  // the token's query as A operands, its head weights by D row
+  bf16x8 qa[KS][HB];
+  float wv[HB][4];
+  const int64_t row = static_cast<int64_t>(b) * a.t_per_seq + min(t, a.t_per_seq - 1);
+  const uint8_t* q = a.q + row * a.n_heads * a.c * 2;
+#pragma unroll
+  for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+    for (int hb = 0; hb < HB; ++hb) {
+      const int h = hb * 16 + col, ch = ks * 32 + grp * 8;
+      const uint8_t* p = (h < a.n_heads && ch < a.c) ? q + (h * a.c + ch) * 2 : g_idx_zero;
+      qa[ks][hb] = as_bf16x8(*reinterpret_cast<const u32x4*>(p));
+    }
+  }
+#pragma unroll
+  for (int hb = 0; hb < HB; ++hb) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int h = hb * 16 + grp * 4 + i;
+      const float* p = h < a.n_heads ? a.w + row * a.n_heads + h : reinterpret_cast<const float*>(g_idx_zero);
+      wv[hb][i] = *p;
+    }
+  }
+  // key staging: thread i holds pieces i, i + 512, ... of a tile
+  u32x4 kreg[kPer];
+  const auto load_tile = [&](int slot) {
+#pragma unroll
+    for (int p = 0; p < kPer; ++p) {
+      const int piece = tid + p * kIrThreads;
+      const int64_t off = src_row[slot][piece / kChunks];
+      const int ch = (piece % kChunks) * 8;
+      const uint8_t* src = (off >= 0 && ch < a.c) ? a.pool + off + ch * 2 : g_idx_zero;
+      kreg[p] = *reinterpret_cast<const u32x4*>(src);
+    }
+  };
+  const auto store_tile = [&](int buf) {
+#pragma unroll
+    for (int p = 0; p < kPer; ++p) {
+      const int piece = tid + p * kIrThreads;
+      *reinterpret_cast<u32x4*>(&keys[buf][piece / kChunks][(piece % kChunks) * 8]) = kreg[p];
+    }
+  };
+  lds_barrier();
+  load_tile(0);
+  store_tile(0);
+  lds_barrier();
+  float* const out = a.scores + row * a.score_stride;
+  // ReLU as the median of x, 0 and infinity, one instruction where a maximum is
+  // two (it quiets its operand first); the compiler must not see the constant
+  float inf = __builtin_huge_valf();
+  asm("" : "+v"(inf));
+  int buf = 0, slot = 0;
+  for (int e0 = e_lo; e0 < e_hi; e0 += kIrTile) {
+    const bool more = e0 + kIrTile < e_hi;  // uniform
+    const int next = slot == 2 ? 0 : slot + 1;
+    int32_t page = 0;
+    if (more) {  // in flight while this tile is multiplied: the next tile's keys, the pages of the one after
+      load_tile(next);
+      page = page_of(e0 + 2 * kIrTile + tid % kIrTile);
+    }
+    // 16-entry blocks in turn: the products of one beside the ReLU and head sum
+    // of the one before and the LDS reads of the next.  The barriers keep that
+    // order (the compiler would chain each accumulator's products, which then
+    // wait for one another).
+    constexpr int kBlocks = kIrTile / 16;
+    bf16x8 kv[2][KS];
+    f32x4 acc[2][HB];
+    float v[kBlocks];
+    const auto read_keys = [&](int j) {
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+        kv[j & 1][ks] = as_bf16x8(*reinterpret_cast<const u32x4*>(&keys[buf][j * 16 + col][ks * 32 + grp * 8]));
+      }
+    };
+    // terms [n0, n1) of block j's head sum: term 4hb + i is head 16hb + 4grp + i
+    const auto head_sum = [&](int j, int n0, int n1) {
+#pragma unroll
+      for (int n = n0; n < n1; ++n) {
+        const float term = __builtin_amdgcn_fmed3f(acc[j & 1][n / 4][n % 4], 0.f, inf);  // ReLU, 0 for NaN
+        v[j] = fmaf(wv[n / 4][n % 4], term, n == 0 ? 0.f : v[j]);
+      }
+    };
+    read_keys(0);
+#pragma unroll
+    for (int j = 0; j < kBlocks; ++j) {
+      if (j + 1 < kBlocks) read_keys(j + 1);
+      __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) {
+#pragma unroll
+        for (int hb = 0; hb < HB; ++hb) {
+          const f32x4 from = ks == 0 ? f32x4{0.f, 0.f, 0.f, 0.f} : acc[j & 1][hb];
+          acc[j & 1][hb] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(qa[ks][hb], kv[j & 1][ks], from, 0, 0, 0);
+          if (j > 0) head_sum(j - 1, (ks * HB + hb) * 4 / KS, (ks * HB + hb + 1) * 4 / KS);
+          __builtin_amdgcn_sched_barrier(0);
+        }
+      }
+    }
+    head_sum(kBlocks - 1, 0, 4 * HB);
+    // heads summed over the lane groups, four entry blocks at once: each
+    // exchange halves the blocks a lane group still holds, so that group g ends
+    // with block g and lane l with entry l of the 64
+    const bool g0 = grp & 1, g1 = grp & 2;
+#pragma unroll
+    for (int r0 = 0; r0 < kIrTile; r0 += kWave) {
+      const float* const w = v + r0 / 16;
+      const float a0 = (g0 ? w[1] : w[0]) + __shfl_xor(g0 ? w[0] : w[1], 16);
+      const float a2 = (g0 ? w[3] : w[2]) + __shfl_xor(g0 ? w[2] : w[3], 16);
+      const float sum = (g1 ? a2 : a0) + __shfl_xor(g1 ? a0 : a2, 32);
+      const int e = e0 + r0 + lane;
+      const bool ok = src_row[slot][r0 + lane] >= 0;
+      if (t < a.t_per_seq && e < e_hi) out[e] = ok ? sum : -__builtin_huge_valf();
+    }
+    if (more) {
+      // the keys' and offsets' last readers passed the barrier of the tile before
+      store_tile(buf ^ 1);
+      if (tid < kIrTile) src_row[next == 2 ? 0 : next + 1][tid] = row_of(e0 + 2 * kIrTile + tid, page);
+      lds_barrier();
+    }
+    slot = next;
+    buf ^= 1;
+  }
+}
+
+template <int HB, int KS>
+void launch_indexer_rows(const IndexerArgs& a, int64_t batch, hipStream_t s) {
+  IndexerRowsArgs ra;
+  ra.a = a;
+  ra.groups = static_cast<int32_t>(ceil_div(a.t_per_seq, kIrTokens));
+  // one workgroup per CU is resident: about four rounds of them, runs of at
+  // least 2 tiles (each workgroup reads its queries once)
+  const int64_t tiles = ceil_div(a.max_entries, kIrTile);
+  const int64_t want = ceil_div(4 * static_cast<int64_t>(device_cus()), batch * ra.groups);
+  const int64_t run = std::max<int64_t>(ceil_div(tiles, want), std::min<int64_t>(tiles, 2));
+  ra.run = static_cast<int32_t>(run * kIrTile);
+  const dim3 grid(static_cast<unsigned>(ceil_div(tiles, run)), static_cast<unsigned>(batch * ra.groups));
+  hipLaunchKernelGGL((k_indexer_scores_rows<HB, KS>), grid, dim3(kIrThreads), 0, s, ra);
 }
 
 }  // namespace skv
@@ -93,6 +290,24 @@ extern "C" int skv_indexer_scores(const void* q, const float* w, const void* idx
   a.n_pages = static_cast<int32_t>(n_pages);
   a.t_per_seq = static_cast<int32_t>(t_per_seq);
   a.max_entries = static_cast<int32_t>(max_entries);
+  // The line: 16 x 16,384 entries and 64 heads take k_indexer_scores 42 us for 4
+  // tokens and 10.5 us for each more, k_indexer_scores_rows 53 us for 4 to 8.
+  if (t_per_seq >= kIrMinTokens) {
+    hipStream_t s = static_cast<hipStream_t>(stream);
+    const int hb = n_heads <= 16 ? 1 : n_heads <= 32 ? 2 : 4, ks = channels <= 32 ? 1 : channels <= 64 ? 2 : 4;
+    switch (hb * 8 + ks) {
+      case 9: launch_indexer_rows<1, 1>(a, batch, s); break;
+      case 10: launch_indexer_rows<1, 2>(a, batch, s); break;
+      case 12: launch_indexer_rows<1, 4>(a, batch, s); break;
+      case 17: launch_indexer_rows<2, 1>(a, batch, s); break;
+      case 18: launch_indexer_rows<2, 2>(a, batch, s); break;
+      case 20: launch_indexer_rows<2, 4>(a, batch, s); break;
+      case 33: launch_indexer_rows<4, 1>(a, batch, s); break;
+      case 34: launch_indexer_rows<4, 2>(a, batch, s); break;
+      default: launch_indexer_rows<4, 4>(a, batch, s); break;
+    }
+    return check_launch(what);
+  }
   const dim3 grid(static_cast<unsigned>(ceil_div(max_entries, kIdxTile)), static_cast<unsigned>(rows));
   hipLaunchKernelGGL(k_indexer_scores, grid, dim3(kIdxThreads), 0, static_cast<hipStream_t>(stream), a);
   return check_launch(what);
