@@ -256,10 +256,10 @@ int skv_topk_select_decode(const float* scores, int64_t score_stride, int64_t ba
                            int64_t out_stride, int32_t* workspace, void* stream);
 
 /* Top-k workspace size in int32 words per row.  workspace == NULL selects one
- * workgroup per row; otherwise each row is cut into 2048-score chunks (one
- * workgroup each, two launches) using rows * skv_topk_workspace_words() words
- * that must be zero before the first call and are left zero by every call.
- * Calls that share a workspace must not overlap. */
+ * workgroup per row; otherwise each row of more than 16384 columns is cut into
+ * 2048-score chunks (one workgroup each, two launches) using rows *
+ * skv_topk_workspace_words() words that must be zero before the first call and
+ * are left zero by every call.  Calls that share a workspace must not overlap. */
 int64_t skv_topk_workspace_words(void);
 
 /* ---- top-k gather -----------------------------------------------------------

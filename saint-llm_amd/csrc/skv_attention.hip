@@ -1164,7 +1164,7 @@ struct StepRank {
       // tie bin over the list capacity: full select of the row, keeping this
       // unit's positions
       auto& fb = *reinterpret_cast<TopkSmemT<kAtThreads>*>(ck);
-      topk_row_emit<kAtThreads>(fb, nullptr, map.scores[0] + static_cast<int64_t>(b) * map.score_stride[0], n_cols,
+      topk_row_emit<kAtThreads>(fb, map.scores[0] + static_cast<int64_t>(b) * map.score_stride[0], n_cols,
                                 n_valid, k, [&](int j, int v) {
                                   if (j >= o0 && j < o1) at_pos[j] = v;
                                 });

@@ -982,7 +982,7 @@ __device__ __forceinline__ void rank_part_body(const skv_decode_desc* __restrict
   if (sel > 0 && flag) {
     // tie bin over the list capacity: full select of the row, keeping this
     // part's positions (each is emitted once)
-    topk_row_emit<kStepThreads>(fb.full, nullptr, map.scores[z] + static_cast<int64_t>(b) * map.score_stride[z],
+    topk_row_emit<kStepThreads>(fb.full, map.scores[z] + static_cast<int64_t>(b) * map.score_stride[z],
                                 n_cols, n_valid, k, [&](int j, int v) {
                                   if (j >= o0 && j < o1) sm.rr.win[j - o0] = make_int2(j, v);
                                 });

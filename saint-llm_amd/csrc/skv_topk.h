@@ -1,10 +1,9 @@
-// Top-k selection of one score row by one 1024-thread workgroup.
+// Top-k selection of one score row by one workgroup.
 //
-// Radix select (8 bits per pass) on order-preserving uint32 keys finds the
+// Radix select (8 bits per pass over the row) on order-preserving uint32 keys finds the
 // threshold key T of rank `sel`; keys > T and the lowest-index keys == T are
-// collected, then ranked by (key descending, index ascending).  Rows with at
-// most kLdsKeys valid scores are staged in LDS, longer rows re-read global
-// memory (L2-resident) on each pass.
+// collected, then ranked by (key descending, index ascending).  It holds for
+// any scores and is the fallback of the faster selections below.
 #pragma once
 
 #include "skv_common.h"
@@ -13,7 +12,6 @@ namespace skv {
 
 constexpr int kTopkThreads = 1024;
 constexpr int kTopkWaves = kTopkThreads / kWave;
-constexpr int kLdsKeys = 28672;  // rows with at most this many valid scores are staged in LDS
 constexpr int kMaxTopK = 2048;
 
 constexpr uint32_t kKeyNaN = 0xffffffffu;
@@ -47,13 +45,11 @@ using TopkSmem = TopkSmemT<kTopkThreads>;
 
 // emit(j, v) for every output position j in [0, k), once each: the sel =
 // min(k, n_cols, n_valid) best of row[0, n_valid) in (score desc, index asc)
-// order, -1 for non-finite picks and ranks >= sel.  `keys` (kLdsKeys words
-// of LDS) stages short rows; nullptr reads global memory on every pass.
-// Every thread of the kThreads-thread workgroup (kThreads >= 256) must call
-// it.
+// order, -1 for non-finite picks and ranks >= sel.  Every thread of the
+// kThreads-thread workgroup (kThreads >= 256) must call it.
 template <int kThreads, class Emit>
-__device__ __forceinline__ void topk_row_emit(TopkSmemT<kThreads>& sm, uint32_t* keys, const float* row,
-                                              int n_cols, int n_valid, int k, Emit emit) {
+__device__ __forceinline__ void topk_row_emit(TopkSmemT<kThreads>& sm, const float* row, int n_cols,
+                                              int n_valid, int k, Emit emit) {
   static_assert(kThreads >= 256 && kThreads % kWave == 0, "topk_row needs >= 256 threads");
   constexpr int kWaves = kThreads / kWave;
   const int tid = threadIdx.x;
@@ -64,12 +60,7 @@ __device__ __forceinline__ void topk_row_emit(TopkSmemT<kThreads>& sm, uint32_t*
   const int sel = min(k_eff, n_valid);
   for (int j = sel + tid; j < k; j += kThreads) emit(j, -1);
   if (sel == 0) return;
-  const bool in_lds = keys != nullptr && n_valid <= kLdsKeys;
-  if (in_lds) {
-    for (int i = tid; i < n_valid; i += kThreads) keys[i] = score_key(row[i]);
-    __syncthreads();
-  }
-  auto key_at = [&](int i) -> uint32_t { return in_lds ? keys[i] : score_key(row[i]); };
+  auto key_at = [&](int i) -> uint32_t { return score_key(row[i]); };
 
   // ---- radix select: the sel-th largest key, 8 bits per pass ---------------
   uint32_t prefix = 0, pmask = 0;
@@ -159,9 +150,166 @@ __device__ __forceinline__ void topk_row_emit(TopkSmemT<kThreads>& sm, uint32_t*
 
 // out[0, k) as topk_row_emit gives it.
 template <int kThreads = kTopkThreads>
-__device__ __forceinline__ void topk_row(TopkSmemT<kThreads>& sm, uint32_t* keys, const float* row,
-                                         int n_cols, int n_valid, int k, int32_t* out) {
-  topk_row_emit<kThreads>(sm, keys, row, n_cols, n_valid, k, [&](int j, int v) { out[j] = v; });
+__device__ __forceinline__ void topk_row(TopkSmemT<kThreads>& sm, const float* row, int n_cols,
+                                         int n_valid, int k, int32_t* out) {
+  topk_row_emit<kThreads>(sm, row, n_cols, n_valid, k, [&](int j, int v) { out[j] = v; });
+}
+
+// ---------------------------------------------------------------------------
+// Selection by value buckets: one workgroup per row, its scores read once into
+// registers (kTbPer per thread; longer rows are read again in each pass).
+//   range   : the smallest and largest finite score, a linear map of the score
+//             to kTbBuckets buckets (monotone: differences, products with a
+//             positive factor and truncation are).  +inf and NaN go to the top
+//             bucket, -inf to bucket 0.
+//   count   : LDS histogram; its sums from the top give every bucket's first
+//             position and the bucket that holds position sel - 1.
+//   scatter : keys of that bucket and above go to their bucket's slots as
+//             64-bit order keys (key << 32 | ~index).
+//   order   : a candidate's position is its bucket's first plus the candidates
+//             of its bucket above it: a few, where the scores spread.
+// The radix select (topk_row_emit) makes four passes of histograms over the row
+// and ranks every winner against every other; it takes the rows whose buckets
+// hold more than kTbMaxBucket candidates, or more than the LDS does (scores
+// that are nearly all equal or hold an outlier far beyond the rest).
+// Latency-bound: 512 picks of 4,096 scores, 2,048 rows 24 us (391 by the radix
+// select, whose 150 KB of LDS kept one row on a CU), one row 9.9 us (48);
+// of 16,384 scores, 500 rows 17.7 us (122).
+// ---------------------------------------------------------------------------
+constexpr int kTbBuckets = 2048;
+constexpr int kTbPer = 16;         // scores per thread held in registers
+constexpr int kTbMaxBucket = 512;  // candidates of one bucket
+constexpr int kTbSlack = 512;      // LDS candidates beyond k
+
+template <int kThreads>
+struct TopkBucketSmem {
+  int scan_lds[17];
+  int threshold[2];  // candidates at and above the threshold bucket, the fullest of those buckets
+  float lo[kThreads / kWave], hi[kThreads / kWave];
+  union {
+    TopkSmemT<kThreads> full;
+    struct {
+      int cursor[kTbBuckets];
+      uint64_t cand[1];  // k + kTbSlack of them
+    } b;
+  } u;
+};
+
+// LDS bytes of topk_row_buckets for k picks.
+template <int kThreads>
+constexpr size_t topk_bucket_lds(int k) {
+  const size_t need = offsetof(TopkBucketSmem<kThreads>, u.b.cand) + sizeof(uint64_t) * (k + kTbSlack);
+  return need > sizeof(TopkBucketSmem<kThreads>) ? need : sizeof(TopkBucketSmem<kThreads>);
+}
+
+// emit(j, v) as topk_row_emit calls it.  kRegs: at most kThreads * kTbPer valid scores.
+template <int kThreads, bool kRegs, class Emit>
+__device__ __forceinline__ void topk_row_buckets(TopkBucketSmem<kThreads>& sm, const float* row, int n_cols, int n_valid,
+                                                 int k, Emit emit) {
+  const int tid = threadIdx.x;
+  n_cols = max(n_cols, 0);
+  n_valid = max(0, min(n_valid, n_cols));
+  const int sel = min(min(k, n_cols), n_valid);
+  for (int j = sel + tid; j < k; j += kThreads) emit(j, -1);
+  if (sel == 0) return;
+  const float inf = __builtin_huge_valf();
+  float f[kTbPer];
+  // each(i, score) over this thread's scores, kTbPer loads in flight at a time
+  const auto each = [&](bool load, auto use) {
+    for (int base = 0; base < n_valid; base += kThreads * kTbPer) {
+      if (load) {
+#pragma unroll
+        for (int q = 0; q < kTbPer; ++q) f[q] = row[min(base + q * kThreads + tid, n_valid - 1)];
+      }
+#pragma unroll
+      for (int q = 0; q < kTbPer; ++q) {
+        if (base + q * kThreads + tid < n_valid) use(base + q * kThreads + tid, f[q]);
+      }
+      if (kRegs) break;
+    }
+  };
+  float lo = inf, hi = -inf;
+  each(true, [&](int, float v) {
+    const bool fin = __builtin_fabsf(v) < inf;
+    lo = fin ? fminf(lo, v) : lo;
+    hi = fin ? fmaxf(hi, v) : hi;
+  });
+  for (int b = tid; b < kTbBuckets; b += kThreads) sm.u.b.cursor[b] = 0;
+  if (tid < 2) sm.threshold[tid] = 0;
+#pragma unroll
+  for (int d = 1; d < kWave; d <<= 1) {
+    lo = fminf(lo, __shfl_xor(lo, d));
+    hi = fmaxf(hi, __shfl_xor(hi, d));
+  }
+  if (tid % kWave == 0) {
+    sm.lo[tid / kWave] = lo;
+    sm.hi[tid / kWave] = hi;
+  }
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < kThreads / kWave; ++w) {
+    lo = fminf(lo, sm.lo[w]);
+    hi = fmaxf(hi, sm.hi[w]);
+  }
+  const float scale = hi > lo ? static_cast<float>(kTbBuckets) / (hi - lo) : 0.f;  // 0 too where the range overflows
+  const auto bucket_of = [&](float v) -> int {
+    const float x = fminf(fmaxf((v - lo) * scale, 0.f), static_cast<float>(kTbBuckets - 1));
+    const int b = static_cast<int>(x);
+    return __builtin_fabsf(v) < inf ? b : (v == -inf ? 0 : kTbBuckets - 1);
+  };
+  each(!kRegs, [&](int, float v) { atomicAdd(&sm.u.b.cursor[bucket_of(v)], 1); });
+  __syncthreads();
+  {
+    constexpr int per = kTbBuckets / kThreads;
+    const int top = kTbBuckets - 1 - tid * per;  // this thread's buckets: top, top - 1, ...
+    int v[per], sum = 0;
+#pragma unroll
+    for (int q = 0; q < per; ++q) {
+      v[q] = sm.u.b.cursor[top - q];
+      sum += v[q];
+    }
+    int tot;
+    int ex = block_exclusive_scan(sum, sm.scan_lds, &tot);  // scores in higher buckets
+    int fullest = 0;
+#pragma unroll
+    for (int q = 0; q < per; ++q) {
+      sm.u.b.cursor[top - q] = ex;
+      if (ex < sel) {
+        fullest = max(fullest, v[q]);
+        if (sel <= ex + v[q]) sm.threshold[0] = ex + v[q];
+      }
+      ex += v[q];
+    }
+    if (fullest > kTbMaxBucket) atomicMax(&sm.threshold[1], fullest);
+  }
+  __syncthreads();
+  const int total = sm.threshold[0];
+  if (__builtin_expect(total > k + kTbSlack || sm.threshold[1] > kTbMaxBucket, 0)) {  // uniform
+    __syncthreads();
+    topk_row_emit<kThreads>(sm.u.full, row, n_cols, n_valid, sel, emit);  // its ranks past sel are written
+    return;
+  }
+  each(!kRegs, [&](int i, float v) {
+    const int b = bucket_of(v);
+    if (sm.u.b.cursor[b] < total) {  // the threshold bucket or above (their slots end at total)
+      const int slot = atomicAdd(&sm.u.b.cursor[b], 1);
+      sm.u.b.cand[slot] = (static_cast<uint64_t>(score_key(v)) << 32) | static_cast<uint32_t>(~i);
+    }
+  });
+  __syncthreads();
+  for (int c = tid; c < total; c += kThreads) {
+    const uint64_t key = sm.u.b.cand[c];
+    const uint32_t hi_key = static_cast<uint32_t>(key >> 32);
+    // the score's bits (every NaN is in the top bucket)
+    const uint32_t bits = (hi_key & 0x80000000u) ? hi_key & 0x7fffffffu : ~hi_key;
+    const int b = bucket_of(hi_key == kKeyNaN ? inf : __uint_as_float(bits));
+    const int first = b == kTbBuckets - 1 ? 0 : sm.u.b.cursor[b + 1];  // the next bucket's end
+    if (first >= sel) continue;
+    const int end = sm.u.b.cursor[b];
+    int rank = 0;
+    for (int j = first; j < end; ++j) rank += sm.u.b.cand[j] > key;
+    if (first + rank < sel) emit(first + rank, key_finite(hi_key) ? static_cast<int>(~static_cast<uint32_t>(key)) : -1);
+  }
 }
 
 // ===========================================================================
@@ -468,7 +616,7 @@ __device__ __forceinline__ void topk_final_row(TopkFinalSmem& sm, const float* r
   int t, above, ties;
   topk_threshold<kTopkThreads>(F.hist, sel, sm.scan_lds, sm.sh, t, above, ties);
   if (ties > kTkTieCap) {
-    topk_row(sm.u.full, nullptr, row, n_cols, n_valid, k, out);
+    topk_row(sm.u.full, row, n_cols, n_valid, k, out);
     __syncthreads();
     topk_clear_ws(ws);
     return;

@@ -15,6 +15,8 @@
 
 namespace skv {
 
+constexpr int64_t kTopkManyRows = 512;  // rows that fill the device with small workgroups
+
 struct TopkArgs {
   const float* scores;
   int64_t stride;
@@ -28,29 +30,6 @@ struct TopkArgs {
   int64_t out_stride;
 };
 
-__global__ __launch_bounds__(kTopkThreads) void k_topk_select(TopkArgs a) {
-  __shared__ TopkSmem sm;
-  __shared__ uint32_t keys[kLdsKeys];
-  const int r = blockIdx.x;
-  int n_cols, n_valid;
-  if (a.lens) {
-    const int L = max(a.lens[r], 0);
-    n_cols = L / a.m;
-    n_valid = L > 0 ? (L - 1) / a.m : 0;
-  } else {
-    n_cols = a.n_cols ? a.n_cols[r] : a.n_cols_uni;
-    n_valid = a.n_valid[r];
-  }
-  topk_row(sm, keys, a.scores + r * a.stride, n_cols, n_valid, a.k, a.out + r * a.out_stride);
-}
-
-// Multi-workgroup form: hist and filter over grid (chunks, rows), final over
-// grid (rows); workspace kTkWsWords int32 per row.
-struct TopkMultiArgs {
-  TopkArgs a;
-  int32_t* ws;
-};
-
 __device__ __forceinline__ void topk_row_dims(const TopkArgs& a, int r, int& n_cols, int& n_valid) {
   if (a.lens) {
     const int L = max(a.lens[r], 0);
@@ -61,6 +40,26 @@ __device__ __forceinline__ void topk_row_dims(const TopkArgs& a, int r, int& n_c
     n_valid = a.n_valid[r];
   }
 }
+
+// One workgroup per row (topk_row_buckets); kRegs: no row has more than
+// kThreads * kTbPer columns.
+template <int kThreads, bool kRegs>
+__global__ __launch_bounds__(kThreads) void k_topk_rows(TopkArgs a) {
+  extern __shared__ char lds[];
+  const int r = blockIdx.x;
+  int n_cols, n_valid;
+  topk_row_dims(a, r, n_cols, n_valid);
+  int32_t* out = a.out + r * a.out_stride;
+  topk_row_buckets<kThreads, kRegs>(*reinterpret_cast<TopkBucketSmem<kThreads>*>(lds), a.scores + r * a.stride, n_cols,
+                                    n_valid, a.k, [&](int j, int v) { out[j] = v; });
+}
+
+// Multi-workgroup form: hist and filter over grid (chunks, rows), final over
+// grid (rows); workspace kTkWsWords int32 per row.
+struct TopkMultiArgs {
+  TopkArgs a;
+  int32_t* ws;
+};
 
 __global__ __launch_bounds__(kTkPartThreads) void k_topk_hist(TopkMultiArgs m) {
   __shared__ TopkHistSmem sm;
@@ -191,6 +190,28 @@ __global__ __launch_bounds__(kGatherThreads) void k_topk_gather(TopkGatherArgs a
 
 using namespace skv;
 
+template <int kThreads, bool kRegs>
+static void launch_topk_rows_as(const TopkArgs& a, int64_t rows, hipStream_t s) {
+  hipLaunchKernelGGL((k_topk_rows<kThreads, kRegs>), dim3(static_cast<unsigned>(rows)), dim3(kThreads),
+                     topk_bucket_lds<kThreads>(a.k), s, a);
+}
+
+// Bounds every row's columns.
+static int64_t topk_cols(const TopkArgs& a) { return (a.lens || a.n_cols) ? a.stride : a.n_cols_uni; }
+
+static void launch_topk_rows(const TopkArgs& a, int64_t rows, hipStream_t s) {
+  const int64_t cols = topk_cols(a);
+  // 256 threads, 16 scores each, where the rows fill the device that way
+  // (2,048 rows of 4,096: 7 on a CU at once); one row alone ends sooner with 1,024
+  if (rows >= kTopkManyRows && cols <= 256 * kTbPer) {
+    launch_topk_rows_as<256, true>(a, rows, s);
+  } else if (cols <= kTopkThreads * kTbPer) {
+    launch_topk_rows_as<kTopkThreads, true>(a, rows, s);
+  } else {
+    launch_topk_rows_as<kTopkThreads, false>(a, rows, s);
+  }
+}
+
 static int launch_topk(const TopkArgs& a, int64_t rows, int32_t* workspace, void* stream,
                        const char* what) {
   if (a.k < 0 || a.k > kMaxTopK) {
@@ -201,8 +222,13 @@ static int launch_topk(const TopkArgs& a, int64_t rows, int32_t* workspace, void
   if (a.stride <= 0) return set_error(SKV_EINVAL, "%s: score_stride must be positive", what);
   if (rows == 0 || a.k == 0) return SKV_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (!workspace) {
-    hipLaunchKernelGGL(k_topk_select, dim3(static_cast<unsigned>(rows)), dim3(kTopkThreads), 0, s, a);
+  // A row of up to 16,384 columns stays in one workgroup's registers, which
+  // beats the three launches whatever the row count (512 of 16,384: 1 row 11.6
+  // against 18.0 us, 500 rows 17.7 against 47.7); longer rows are read three
+  // times by one workgroup (1,024 of 65,536: 31.0 against 27.5 us, of 262,144:
+  // 99 against 31) and take the launches where the caller gives a workspace.
+  if (!workspace || topk_cols(a) <= kTopkThreads * kTbPer) {
+    launch_topk_rows(a, rows, s);
     return check_launch(what);
   }
   TopkMultiArgs m{a, workspace};

@@ -82,8 +82,8 @@ def indexer_topk(q_indexer: torch.Tensor, head_weights: torch.Tensor, k_indexer_
     n_valid = torch.clamp(q_pos // m, max=n_blocks).to(torch.int32).repeat(b)
     rows = b * t_new
     out = torch.empty(rows, k_eff, dtype=torch.int32, device=dev)
-    # long rows are spread over several workgroups through a zeroed workspace
-    ws = ops.topk_workspace(rows, dev) if n_blocks > 4096 else None
+    # rows past 16384 columns are spread over several workgroups through a zeroed workspace
+    ws = ops.topk_workspace(rows, dev) if n_blocks > 16384 else None
     ops.topk_select(scores.view(rows, n_blocks), n_valid, n_blocks, k_eff, out, ws)
     return out.view(b, t_new, k_eff).long()
 
