@@ -860,8 +860,15 @@ __global__ __launch_bounds__(256) void k_attn_merge_q(MergeArgs a) {
   }
 }
 
+}  // namespace skv
+
+#include "skv_attn_rows.h"
+
+namespace skv {
+
 struct AttnPlan {
   int n_cu, n_wu, n_hg, nks;
+  bool by_rows;  // one workgroup per (query row, head group): k_attn_rows, no workspace
   int64_t rows;  // query rows: batch x query tokens per sequence
   int64_t nq, ring, win_row;
   int64_t ws_bytes;
@@ -958,6 +965,12 @@ int attn_plan(const skv_attention_desc* d, AttnPlan& p) {
   p.n_wu = static_cast<int>(n_wu);
   const int64_t units = p.rows * (n_cu + n_wu) * p.n_hg;
   if (units >= (1 << 30)) return set_error(SKV_EINVAL, "%s: too many workgroups", what);
+  // From a row per two CUs on a row is not split further (its two branches fill
+  // the device), and one workgroup for both of them is faster than two units and a
+  // merge (512 picks and a window of 128, 64 heads x 576: 128 rows 58 against 67 us,
+  // 256 rows 60 against 115, 512 rows 114 against 216); wider windows' scores do
+  // not fit its LDS.
+  p.by_rows = d->splits <= 0 && d->window <= kRowsMaxWindow && 2 * p.rows * p.n_hg >= device_cus();
   p.ws_bytes = units * kAtHeads * (2 * static_cast<int64_t>(sizeof(float)) + d->head_dim * 2);  // (max, sum) fp32, O bf16
   return SKV_OK;
 }
@@ -1636,6 +1649,20 @@ extern "C" int skv_decode_attention(const skv_attention_desc* d, void* workspace
   a.fused = 0;
   a.xcds = device_xcds();
   hipStream_t s = static_cast<hipStream_t>(stream);
+  if (p.by_rows) {
+    const AttnRowsArgs ra{a, d->out, d->sink, d->kind == SKV_LAYER_HCA};
+    const dim3 rows(static_cast<unsigned>(a.xcds * ceil_div(p.rows * p.n_hg, a.xcds)));
+    if (a.fp8_main > 0) {
+      hipLaunchKernelGGL((k_attn_rows<18, true>), rows, dim3(kAtThreads), 0, s, ra);
+    } else if (p.nks == 4) {
+      hipLaunchKernelGGL((k_attn_rows<4, false>), rows, dim3(kAtThreads), 0, s, ra);
+    } else if (p.nks == 16) {
+      hipLaunchKernelGGL((k_attn_rows<16, false>), rows, dim3(kAtThreads), 0, s, ra);
+    } else {
+      hipLaunchKernelGGL((k_attn_rows<18, false>), rows, dim3(kAtThreads), 0, s, ra);
+    }
+    return check_launch(what);
+  }
   const dim3 grid(static_cast<unsigned>(a.xcds * ceil_div(p.rows, a.xcds) * (p.n_cu + p.n_wu) * p.n_hg));
   if (a.fp8_main > 0) {
     hipLaunchKernelGGL((k_attn_part<18, true>), grid, dim3(kAtThreads), 0, s, a);
