@@ -295,6 +295,20 @@ int skv_indexer_scores(const void* q, const float* w, const void* idx_pool, int6
                        int64_t t_per_seq, int64_t n_heads, int64_t channels, int64_t max_entries,
                        void* stream);
 
+/* The picks of a chunk of t_new query tokens per sequence over contiguous
+ * compressed indexer keys (csa.py:405-422): scores as skv_indexer_scores, then
+ * the top-k of what each token sees.  q: bf16 [batch, t_new, n_heads,
+ * channels]; w: fp32 [batch, t_new, n_heads]; keys: bf16 [batch, key_rows,
+ * channels], of which the first n_blocks rows count; token t sees the entries
+ * s < min((cache_offset + t) / m, n_blocks).  scores: scratch, fp32 [batch *
+ * t_new, n_blocks]; out_idx: int64 [batch * t_new, k], the visible entries by
+ * descending score (ties: lower entry first), -1 for a score that is not finite
+ * and past the visible.  n_blocks <= 16384, positions below 2^31; otherwise the
+ * limits of skv_indexer_scores and skv_topk_select. */
+int skv_indexer_topk(const void* q, const float* w, const void* keys, int64_t key_rows, float* scores,
+                     int64_t* out_idx, int64_t batch, int64_t t_new, int64_t n_heads, int64_t channels,
+                     int64_t n_blocks, int64_t cache_offset, int64_t m, int64_t k, void* stream);
+
 /* ---- eviction and compaction --------------------------------------------------
  * skv_release: push every page of each sequence with release_mask[b] != 0 back
  * on the free stack (ascending b; within b from the last logical page to the

@@ -20,15 +20,23 @@ struct IndexerArgs {
   const uint8_t* q;  // [rows, H, c] bf16, rows = batch * t_per_seq
   const float* w;    // [rows, H]
   const uint8_t* pool;  // [n_pages, block_size, c] bf16
-  const int32_t* block_table;
-  const int32_t* n_entries;
+  const int32_t* block_table;  // nullptr: a chunk's keys, sequence b's in page b
+  const int32_t* n_entries;    // nullptr with it: max_entries
   float* scores;  // [rows, score_stride]
   int64_t score_stride;
   int32_t bt_stride;
   int32_t n_heads, c, block_size, n_pages, t_per_seq, max_entries;
+  int32_t offset, m;  // a chunk's token t sees the entries below (offset + t) / m
 };
 
+// Entries that token t of sequence b is scored against.
+template <bool kChunk>
+__device__ __forceinline__ int indexer_entries(const IndexerArgs& a, int b, int t) {
+  return min(kChunk ? (a.offset + t) / a.m : a.n_entries[b], a.max_entries);
+}
+
 // One workgroup per (tile of kIdxTile entries, query row).
+template <bool kChunk>
 __global__ __launch_bounds__(kIdxThreads, 2) void k_indexer_scores(IndexerArgs a) {
   __shared__ IndexerSmem sm;
   const int row = blockIdx.y;  // query row
@@ -36,16 +44,17 @@ __global__ __launch_bounds__(kIdxThreads, 2) void k_indexer_scores(IndexerArgs a
   const IndexerRow r{a.q + static_cast<int64_t>(row) * a.n_heads * a.c * 2,
                      a.w + static_cast<int64_t>(row) * a.n_heads,
                      a.pool,
-                     a.block_table + static_cast<int64_t>(b) * a.bt_stride,
+                     kChunk ? nullptr : a.block_table + static_cast<int64_t>(b) * a.bt_stride,
                      a.bt_stride,
                      a.block_size,
                      a.n_pages,
                      a.n_heads,
-                     a.c};
+                     a.c,
+                     b};
   float* out = a.scores + static_cast<int64_t>(row) * a.score_stride;
-  indexer_tile(
+  indexer_tile<!kChunk>(
       sm, r, static_cast<int>(blockIdx.x),
-      [&] { return min(a.n_entries[b], a.max_entries); },  // the grid covers max_entries
+      [&] { return indexer_entries<kChunk>(a, b, row - b * a.t_per_seq); },  // the grid covers max_entries
       [&](int e, float v) { out[e] = v; });
 }
 
@@ -79,7 +88,8 @@ __device__ __align__(16) uint8_t g_idx_zero[16];
 
 // HB: 16-head blocks, KS: 32-channel steps (heads and channels past the
 // query's are zero in both operands).
-template <int HB, int KS>
+// kChunk: the entries up to those that the workgroup's last token sees.
+template <int HB, int KS, bool kChunk>
 __global__ __launch_bounds__(kIrThreads, 2) void k_indexer_scores_rows(IndexerRowsArgs ra) {
   const IndexerArgs& a = ra.a;
   constexpr int kRow = 32 * KS + 8;  // LDS row of a key (16 bytes of pad: distinct banks)
@@ -92,13 +102,14 @@ __global__ __launch_bounds__(kIrThreads, 2) void k_indexer_scores_rows(IndexerRo
   const int wave = __builtin_amdgcn_readfirstlane(tid) / kWave;
   const int col = lane & 15, grp = lane >> 4;
   const int b = blockIdx.y / ra.groups;
-  const int t = (blockIdx.y - b * ra.groups) * kIrTokens + wave;  // this wave's token
-  const int n_ent = min(a.n_entries[b], a.max_entries);
+  const int t0 = (blockIdx.y - b * ra.groups) * kIrTokens;
+  const int t = t0 + wave;  // this wave's token
+  const int n_ent = indexer_entries<kChunk>(a, b, min(t0 + kIrTokens, a.t_per_seq) - 1);
   const int e_lo = blockIdx.x * ra.run, e_hi = min(n_ent, e_lo + ra.run);
   if (e_lo >= e_hi) return;  // uniform
   const int32_t* bt_row = a.block_table + static_cast<int64_t>(b) * a.bt_stride;
   // entry e's page (loaded a tile ahead of its key) and its key's offset
-  const auto page_of = [&](int e) { return bt_row[min(static_cast<int>(udiv24(e, a.block_size)), a.bt_stride - 1)]; };
+  const auto page_of = [&](int e) { return kChunk ? b : bt_row[min(static_cast<int>(udiv24(e, a.block_size)), a.bt_stride - 1)]; };
   const auto row_of = [&](int e, int32_t page) -> int64_t {
     const int pi = static_cast<int>(udiv24(e, a.block_size));
     const bool ok = e < e_hi && pi < a.bt_stride && page >= 0 && page < a.n_pages;
@@ -229,7 +240,7 @@ __global__ __launch_bounds__(kIrThreads, 2) void k_indexer_scores_rows(IndexerRo
   }
 }
 
-template <int HB, int KS>
+template <int HB, int KS, bool kChunk>
 void launch_indexer_rows(const IndexerArgs& a, int64_t batch, hipStream_t s) {
   IndexerRowsArgs ra;
   ra.a = a;
@@ -241,7 +252,62 @@ void launch_indexer_rows(const IndexerArgs& a, int64_t batch, hipStream_t s) {
   const int64_t run = std::max<int64_t>(ceil_div(tiles, want), std::min<int64_t>(tiles, 2));
   ra.run = static_cast<int32_t>(run * kIrTile);
   const dim3 grid(static_cast<unsigned>(ceil_div(tiles, run)), static_cast<unsigned>(batch * ra.groups));
-  hipLaunchKernelGGL((k_indexer_scores_rows<HB, KS>), grid, dim3(kIrThreads), 0, s, ra);
+  hipLaunchKernelGGL((k_indexer_scores_rows<HB, KS, kChunk>), grid, dim3(kIrThreads), 0, s, ra);
+}
+
+template <bool kChunk>
+void launch_indexer(const IndexerArgs& a, int64_t batch, hipStream_t s) {
+  // The line: 16 x 16,384 entries and 64 heads take k_indexer_scores 42 us for 4
+  // tokens and 10.5 us for each more, k_indexer_scores_rows 53 us for 4 to 8.
+  if (a.t_per_seq >= kIrMinTokens) {
+    const int hb = a.n_heads <= 16 ? 1 : a.n_heads <= 32 ? 2 : 4, ks = a.c <= 32 ? 1 : a.c <= 64 ? 2 : 4;
+    switch (hb * 8 + ks) {
+      case 9: launch_indexer_rows<1, 1, kChunk>(a, batch, s); break;
+      case 10: launch_indexer_rows<1, 2, kChunk>(a, batch, s); break;
+      case 12: launch_indexer_rows<1, 4, kChunk>(a, batch, s); break;
+      case 17: launch_indexer_rows<2, 1, kChunk>(a, batch, s); break;
+      case 18: launch_indexer_rows<2, 2, kChunk>(a, batch, s); break;
+      case 20: launch_indexer_rows<2, 4, kChunk>(a, batch, s); break;
+      case 33: launch_indexer_rows<4, 1, kChunk>(a, batch, s); break;
+      case 34: launch_indexer_rows<4, 2, kChunk>(a, batch, s); break;
+      default: launch_indexer_rows<4, 4, kChunk>(a, batch, s); break;
+    }
+    return;
+  }
+  const dim3 grid(static_cast<unsigned>(ceil_div(a.max_entries, kIdxTile)), static_cast<unsigned>(batch * a.t_per_seq));
+  hipLaunchKernelGGL(k_indexer_scores<kChunk>, grid, dim3(kIdxThreads), 0, s, a);
+}
+
+int indexer_check_query(const char* what, int64_t n_heads, int64_t channels) {
+  if (n_heads < 1 || n_heads > 16 * kIdxMaxHB) {
+    return set_error(SKV_EINVAL, "%s: n_heads must be in [1, %d]; got %lld", what, 16 * kIdxMaxHB,
+                     (long long)n_heads);
+  }
+  if (channels < 8 || channels > 32 * kIdxMaxKS || channels % 8) {
+    return set_error(SKV_EINVAL, "%s: channels must be a multiple of 8 in [8, %d]; got %lld", what,
+                     32 * kIdxMaxKS, (long long)channels);
+  }
+  return SKV_OK;
+}
+
+int launch_indexer_chunk(const IndexerChunk& x, hipStream_t s) {
+  IndexerArgs a{};
+  a.q = static_cast<const uint8_t*>(x.q);
+  a.w = x.w;
+  a.pool = static_cast<const uint8_t*>(x.keys);
+  a.scores = x.scores;
+  a.score_stride = x.n_blocks;
+  a.bt_stride = 1;
+  a.n_heads = static_cast<int32_t>(x.n_heads);
+  a.c = static_cast<int32_t>(x.channels);
+  a.block_size = static_cast<int32_t>(x.key_rows);
+  a.n_pages = static_cast<int32_t>(x.batch);
+  a.t_per_seq = static_cast<int32_t>(x.t_new);
+  a.max_entries = static_cast<int32_t>(x.n_blocks);
+  a.offset = static_cast<int32_t>(x.offset);
+  a.m = static_cast<int32_t>(x.m);
+  launch_indexer<true>(a, x.batch, s);
+  return check_launch("skv_indexer_topk");
 }
 
 }  // namespace skv
@@ -259,14 +325,7 @@ extern "C" int skv_indexer_scores(const void* q, const float* w, const void* idx
   if (!q || !w || !idx_pool || !block_table || !n_entries || !scores) {
     return set_error(SKV_EINVAL, "%s: NULL pointer", what);
   }
-  if (n_heads < 1 || n_heads > 16 * kIdxMaxHB) {
-    return set_error(SKV_EINVAL, "%s: n_heads must be in [1, %d]; got %lld", what, 16 * kIdxMaxHB,
-                     (long long)n_heads);
-  }
-  if (channels < 8 || channels > 32 * kIdxMaxKS || channels % 8) {
-    return set_error(SKV_EINVAL, "%s: channels must be a multiple of 8 in [8, %d]; got %lld", what,
-                     32 * kIdxMaxKS, (long long)channels);
-  }
+  if (const int rc = indexer_check_query(what, n_heads, channels)) return rc;
   if (block_size <= 0 || n_pages <= 0 || n_pages > 0x7fffffff || bt_stride <= 0 || bt_stride >= (1 << 24)) {
     return set_error(SKV_EINVAL, "%s: bad page geometry", what);
   }
@@ -290,25 +349,6 @@ extern "C" int skv_indexer_scores(const void* q, const float* w, const void* idx
   a.n_pages = static_cast<int32_t>(n_pages);
   a.t_per_seq = static_cast<int32_t>(t_per_seq);
   a.max_entries = static_cast<int32_t>(max_entries);
-  // The line: 16 x 16,384 entries and 64 heads take k_indexer_scores 42 us for 4
-  // tokens and 10.5 us for each more, k_indexer_scores_rows 53 us for 4 to 8.
-  if (t_per_seq >= kIrMinTokens) {
-    hipStream_t s = static_cast<hipStream_t>(stream);
-    const int hb = n_heads <= 16 ? 1 : n_heads <= 32 ? 2 : 4, ks = channels <= 32 ? 1 : channels <= 64 ? 2 : 4;
-    switch (hb * 8 + ks) {
-      case 9: launch_indexer_rows<1, 1>(a, batch, s); break;
-      case 10: launch_indexer_rows<1, 2>(a, batch, s); break;
-      case 12: launch_indexer_rows<1, 4>(a, batch, s); break;
-      case 17: launch_indexer_rows<2, 1>(a, batch, s); break;
-      case 18: launch_indexer_rows<2, 2>(a, batch, s); break;
-      case 20: launch_indexer_rows<2, 4>(a, batch, s); break;
-      case 33: launch_indexer_rows<4, 1>(a, batch, s); break;
-      case 34: launch_indexer_rows<4, 2>(a, batch, s); break;
-      default: launch_indexer_rows<4, 4>(a, batch, s); break;
-    }
-    return check_launch(what);
-  }
-  const dim3 grid(static_cast<unsigned>(ceil_div(max_entries, kIdxTile)), static_cast<unsigned>(rows));
-  hipLaunchKernelGGL(k_indexer_scores, grid, dim3(kIdxThreads), 0, static_cast<hipStream_t>(stream), a);
+  launch_indexer<false>(a, batch, static_cast<hipStream_t>(stream));
   return check_launch(what);
 }

@@ -37,6 +37,20 @@ __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast
 
 // The query row in LDS, heads padded to 64 and channels to 128 with zeros;
 // rows of 272 bytes put the 16 lanes that read one A operand on distinct banks.
+// A chunk of t_new query tokens per sequence scored against the n_blocks
+// contiguous keys of each sequence (key_rows rows apart), token t against those
+// below (offset + t) / m.  scores: [batch * t_new, n_blocks].
+struct IndexerChunk {
+  const void* q;     // [batch, t_new, n_heads, channels] bf16
+  const float* w;    // [batch, t_new, n_heads]
+  const void* keys;  // [batch, key_rows, channels] bf16
+  float* scores;
+  int64_t batch, t_new, n_heads, channels, key_rows, n_blocks, offset, m;
+};
+
+int indexer_check_query(const char* what, int64_t n_heads, int64_t channels);
+int launch_indexer_chunk(const IndexerChunk& x, hipStream_t s);
+
 struct IndexerSmem {
   alignas(16) uint16_t q[16 * kIdxMaxHB][kIdxQRow];
 };
@@ -46,8 +60,9 @@ struct IndexerRow {
   const uint8_t* q;       // [n_heads, c] bf16
   const float* w;         // [n_heads]
   const uint8_t* pool;    // [n_pages, block_size, c] bf16
-  const int32_t* bt_row;  // the sequence's block-table row
+  const int32_t* bt_row;  // the sequence's block-table row, nullptr: its only page is `page`
   int bt_stride, block_size, n_pages, n_heads, c;
+  int page = 0;
 };
 
 // Scores of entries [tile * kIdxTile, +kIdxTile) below count(): out(e, v) is
@@ -57,7 +72,7 @@ struct IndexerRow {
 // slots, the query and the weights), so that its own loads overlap them.
 // Returns false (uniformly, before any barrier) when the tile lies past the
 // count; otherwise every thread passes one __syncthreads.
-template <class Count, class Out>
+template <bool kPaged = true, class Count, class Out>
 __device__ __forceinline__ bool indexer_tile(IndexerSmem& sm, const IndexerRow& r, int tile, Count count,
                                              Out out) {
   const int tid = threadIdx.x;
@@ -70,7 +85,7 @@ __device__ __forceinline__ bool indexer_tile(IndexerSmem& sm, const IndexerRow& 
 #pragma unroll
   for (int j = 0; j < kIdxCols; ++j) {
     pi[j] = static_cast<int>(udiv24(e0 + 16 * j, r.block_size));
-    page[j] = r.bt_row[min(pi[j], r.bt_stride - 1)];
+    page[j] = kPaged ? r.bt_row[min(pi[j], r.bt_stride - 1)] : r.page;
   }
   constexpr int kQChunks = 16 * kIdxMaxHB * (32 * kIdxMaxKS / 8);  // 16-byte pieces of the padded query
   u32x4 qv[kQChunks / kIdxThreads];

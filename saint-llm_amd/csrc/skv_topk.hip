@@ -11,6 +11,7 @@
 //   dequant_from_fp8 (quant/reference.py:114-116): code * scale, then bf16.
 // Order of equal scores: ascending index (a total order; torch leaves ties
 // unspecified).
+#include "skv_indexer_tile.h"
 #include "skv_topk.h"
 
 namespace skv {
@@ -28,6 +29,9 @@ struct TopkArgs {
   int k;
   int32_t* out;
   int64_t out_stride;
+  int64_t* out64;         // not nullptr: the rows' picks go here
+  int t_new;              // > 0 (a chunk's query tokens): row r sees (offset + r % t_new) / m columns
+  int offset;
 };
 
 __device__ __forceinline__ void topk_row_dims(const TopkArgs& a, int r, int& n_cols, int& n_valid) {
@@ -35,6 +39,9 @@ __device__ __forceinline__ void topk_row_dims(const TopkArgs& a, int r, int& n_c
     const int L = max(a.lens[r], 0);
     n_cols = L / a.m;
     n_valid = L > 0 ? (L - 1) / a.m : 0;
+  } else if (a.t_new > 0) {
+    n_cols = a.n_cols_uni;
+    n_valid = (a.offset + r % a.t_new) / a.m;
   } else {
     n_cols = a.n_cols ? a.n_cols[r] : a.n_cols_uni;
     n_valid = a.n_valid[r];
@@ -49,9 +56,15 @@ __global__ __launch_bounds__(kThreads) void k_topk_rows(TopkArgs a) {
   const int r = blockIdx.x;
   int n_cols, n_valid;
   topk_row_dims(a, r, n_cols, n_valid);
-  int32_t* out = a.out + r * a.out_stride;
+  const int64_t at = r * a.out_stride;
   topk_row_buckets<kThreads, kRegs>(*reinterpret_cast<TopkBucketSmem<kThreads>*>(lds), a.scores + r * a.stride, n_cols,
-                                    n_valid, a.k, [&](int j, int v) { out[j] = v; });
+                                    n_valid, a.k, [&](int j, int v) {
+                                      if (a.out64) {
+                                        a.out64[at + j] = v;
+                                      } else {
+                                        a.out[at + j] = v;
+                                      }
+                                    });
 }
 
 // Multi-workgroup form: hist and filter over grid (chunks, rows), final over
@@ -276,6 +289,47 @@ extern "C" int skv_topk_select_decode(const float* scores, int64_t score_stride,
   a.out = out_idx;
   a.out_stride = out_stride;
   return launch_topk(a, batch, workspace, stream, "skv_topk_select_decode");
+}
+
+// The chunk's scores and picks in two launches: what each token sees is worked out
+// in the kernels, the keys are read where they lie and entries past the last token
+// of a workgroup are not scored.  With the mask, the keys' copy and the picks'
+// widening in launches of their own a single token over 250 entries took 83 us,
+// bound by them; now 19.  2,048 tokens from position 15 on, 64 heads: 39 us (327
+// with all entries scored and the radix selection); from 14,336 on 171.
+extern "C" int skv_indexer_topk(const void* q, const float* w, const void* keys, int64_t key_rows, float* scores,
+                                int64_t* out_idx, int64_t batch, int64_t t_new, int64_t n_heads, int64_t channels,
+                                int64_t n_blocks, int64_t cache_offset, int64_t m, int64_t k, void* stream) {
+  const char* what = "skv_indexer_topk";
+  if (batch < 0 || t_new < 0 || n_blocks < 0 || k < 0) return set_error(SKV_EINVAL, "%s: negative size", what);
+  if (batch == 0 || t_new == 0 || n_blocks == 0 || k == 0) return SKV_OK;
+  if (!q || !w || !keys || !scores || !out_idx) return set_error(SKV_EINVAL, "%s: NULL pointer", what);
+  if (const int rc = indexer_check_query(what, n_heads, channels)) return rc;
+  if (n_blocks > kTopkThreads * kTbPer || key_rows < n_blocks || key_rows >= (1 << 24)) {
+    return set_error(SKV_EINVAL, "%s: need n_blocks <= %d and n_blocks <= key_rows < 2^24", what, kTopkThreads * kTbPer);
+  }
+  if (m < 1 || m > INT32_MAX || cache_offset < 0 || cache_offset > INT32_MAX || t_new > INT32_MAX - cache_offset) {
+    return set_error(SKV_EINVAL, "%s: need m >= 1 and positions below 2^31", what);
+  }
+  if (batch > 65535 || t_new > 65535 || batch * t_new > 65535) {
+    return set_error(SKV_EINVAL, "%s: at most 65535 query rows", what);
+  }
+  if (k > kMaxTopK) return set_error(SKV_EINVAL, "%s: k must be in [0, %d]; got %lld", what, kMaxTopK, (long long)k);
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const IndexerChunk x{q, w, keys, scores, batch, t_new, n_heads, channels, key_rows, n_blocks, cache_offset, m};
+  if (const int rc = launch_indexer_chunk(x, s)) return rc;
+  TopkArgs a{};
+  a.scores = scores;
+  a.stride = n_blocks;
+  a.n_cols_uni = static_cast<int>(n_blocks);
+  a.m = static_cast<int>(m);
+  a.k = static_cast<int>(k);
+  a.out64 = out_idx;
+  a.out_stride = k;
+  a.t_new = static_cast<int>(t_new);
+  a.offset = static_cast<int>(cache_offset);
+  launch_topk_rows(a, batch * t_new, s);
+  return check_launch(what);
 }
 
 extern "C" int skv_topk_gather(void* dst, const void* pool, int64_t entry_bytes, int64_t block_size,

@@ -61,13 +61,14 @@ def indexer_topk(q_indexer: torch.Tensor, head_weights: torch.Tensor, k_indexer_
     position q iff s * m + m - 1 < q (csa.py:411-415); a row's picks are its
     visible entries by descending score (ties: lower entry first), and a pick
     whose score is not finite (a masked entry, NaN, +-inf) is -1
-    (csa.py:420-422).  The scores come from skv_indexer_scores, the picks from
+    (csa.py:420-422).  Up to 16384 entries both come from skv_indexer_topk,
+    past them the scores from skv_indexer_scores and the picks from
     skv_topk_select (one row per query token).
     """
     if q_indexer.dim() != 4 or head_weights.dim() != 3 or k_indexer_comp.dim() != 3:
         raise ValueError("q_indexer must be (B, t_new, H, c), head_weights (B, t_new, H), "
                          "k_indexer_comp (B, n_blocks, c)")
-    b, t_new, _, c = q_indexer.shape
+    b, t_new, h, c = q_indexer.shape
     if total_len - cache_offset != t_new or cache_offset < 0:
         raise ValueError(f"total_len - cache_offset must equal t_new={t_new}; got {cache_offset}..{total_len}")
     if m <= 0 or top_k < 0 or n_blocks < 0 or n_blocks > k_indexer_comp.shape[1]:
@@ -76,13 +77,23 @@ def indexer_topk(q_indexer: torch.Tensor, head_weights: torch.Tensor, k_indexer_
     k_eff = min(top_k, n_blocks)
     if k_eff == 0 or b == 0 or t_new == 0:
         return torch.full((b, t_new, k_eff), -1, dtype=torch.long, device=dev)
+    if k_indexer_comp.shape[0] != b or k_indexer_comp.shape[2] != c or tuple(head_weights.shape) != (b, t_new, h):
+        raise ValueError("q_indexer, k_indexer_comp and head_weights disagree on B, T, H or c")
+    if n_blocks <= 16384 and total_len < 2 ** 31:
+        keys = k_indexer_comp
+        if keys.dtype != torch.bfloat16 or not keys.is_contiguous() or keys.data_ptr() % 16 or keys.shape[1] >= 1 << 24:
+            keys = keys[:, :n_blocks].to(torch.bfloat16).contiguous()
+        out = torch.empty(b, t_new, k_eff, dtype=torch.long, device=dev)
+        # an m past every position shows nothing, whatever its value
+        return ops.indexer_topk_chunk(q_indexer.to(torch.bfloat16).contiguous(), head_weights.float().contiguous(),
+                                      keys, n_blocks, int(cache_offset), min(int(m), int(total_len) + 1), out)
     scores = lightning_indexer_scores(q_indexer, k_indexer_comp[:, :n_blocks], head_weights)  # (B, t_new, n)
     # visible entries of the query at position q: s < floor(q / m) (s * m + m - 1 < q)
     q_pos = torch.arange(cache_offset, total_len, device=dev, dtype=torch.int64)
     n_valid = torch.clamp(q_pos // m, max=n_blocks).to(torch.int32).repeat(b)
     rows = b * t_new
     out = torch.empty(rows, k_eff, dtype=torch.int32, device=dev)
-    # rows past 16384 columns are spread over several workgroups through a zeroed workspace
+    # more than 16384 columns are spread over several workgroups through a zeroed workspace
     ws = ops.topk_workspace(rows, dev) if n_blocks > 16384 else None
     ops.topk_select(scores.view(rows, n_blocks), n_valid, n_blocks, k_eff, out, ws)
     return out.view(b, t_new, k_eff).long()

@@ -599,6 +599,35 @@ def indexer_scores(q: torch.Tensor, w: torch.Tensor, idx_pool: torch.Tensor, blo
     return out
 
 
+def indexer_topk_chunk(q: torch.Tensor, w: torch.Tensor, keys: torch.Tensor, n_blocks: int, cache_offset: int,
+                       m: int, out: torch.Tensor) -> torch.Tensor:
+    """out[b, t]: the picks of query token t of sequence b among its visible
+    entries s < min((cache_offset + t) // m, n_blocks), -1 past them.
+
+    q: bf16 [B, T, H, c]; w: fp32 [B, T, H]; keys: bf16 [B, >= n_blocks, c],
+    n_blocks <= 16384; out: int64 [B, T, k]; all contiguous.
+    """
+    _require_gpu(q, "q")
+    if q.dtype != torch.bfloat16 or q.dim() != 4 or not q.is_contiguous():
+        raise ValueError("q must be a contiguous bf16 [B, T, H, c] tensor")
+    batch, t, heads, c = q.shape
+    _require_gpu(w, "w")
+    if w.dtype != torch.float32 or tuple(w.shape) != (batch, t, heads) or not w.is_contiguous():
+        raise ValueError(f"w must be a contiguous fp32 [{batch}, {t}, {heads}] tensor")
+    _require_gpu(keys, "keys")
+    if keys.dtype != torch.bfloat16 or keys.dim() != 3 or keys.shape[0] != batch or keys.shape[2] != c or \
+            keys.shape[1] < n_blocks or not keys.is_contiguous():
+        raise ValueError(f"keys must be a contiguous bf16 [{batch}, >= {n_blocks}, {c}] tensor")
+    _require_gpu(out, "out")
+    if out.dtype != torch.int64 or out.dim() != 3 or tuple(out.shape[:2]) != (batch, t) or not out.is_contiguous():
+        raise ValueError(f"out must be a contiguous int64 [{batch}, {t}, k] tensor")
+    scores = torch.empty(batch * t * n_blocks, dtype=torch.float32, device=q.device)
+    _lib.call("skv_indexer_topk", q.data_ptr(), w.data_ptr(), keys.data_ptr(), keys.shape[1], scores.data_ptr(),
+              out.data_ptr(), batch, t, heads, c, n_blocks, cache_offset, m, out.shape[2],
+              _lib.stream_handle(q.device))
+    return out
+
+
 # ---------------------------------------------------------------------------
 # Eviction and compaction
 # ---------------------------------------------------------------------------
