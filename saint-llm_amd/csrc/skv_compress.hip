@@ -52,10 +52,11 @@ struct CompressArgs {
 // per workgroup); one of 128 takes all 16 lane groups, 8 tokens each.
 // HBM-bound: c and z rows are read once.  One wave folding an entry's tokens one
 // after another, with a memory round trip each, took 1.45 us per token.  4
-// sequences of 6,700-8,192 tokens x 576 bf16 channels: entries of 4 tokens 25.4 us
-// (3.0 TB/s; the call averaged 247 us before), of 128 tokens 26 us; 16 x 8,192
-// tokens 86 us (3.95 TB/s, a plain copy 4.9); two sequences of 95 and 300 tokens 5.5
-// and, with blocks of 128, 8.3 us (186 before).
+// sequences of 6,700-8,192 tokens x 576 bf16 channels: entries of 4 tokens 33 us
+// (2.6 TB/s; the call averaged 247 us before; 25 with the weights of a turn taken
+// against its max at once, which moves the last bits of the sums and so codes of
+// fp8 entries), of 128 tokens 26 us; 16 x 8,192 tokens in entries of 4 110 us; two
+// sequences of 95 and 300 tokens 5.5 and, with blocks of 128, 8.3 us (186 before).
 constexpr int kCmThreads = 256;
 constexpr int kCmWaves = kCmThreads / kWave;
 constexpr int kCmLanes = 16;                         // lanes per 128-channel token row
@@ -99,7 +100,7 @@ struct RawRow {
 // Tokens first + slice + stride * i < p1 of entry e (sequence b) folded into
 // st.  Every load of a turn is issued before any is used (left to itself the
 // compiler waits for each row in turn: 14.8 us for a call of a few entries).
-template <class Row>
+template <class Row, bool kSerial>
 __device__ __forceinline__ void fold_tokens(PoolLane& st, const CompressArgs& a, int b, int first_new, int e, int first,
                                             int p1, int slice, int stride, int grp) {
   typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // bias is 4-byte aligned
@@ -122,11 +123,11 @@ __device__ __forceinline__ void fold_tokens(PoolLane& st, const CompressArgs& a,
       br[u][1] = bp[1];
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (__ballot(!live[kCmFold - 1])) {  // tokens past the end: value -inf, row 0
+    if (__ballot(!live[kCmFold - 1])) {  // tokens past the end: value -inf, row -0: nothing is added
 #pragma unroll
       for (int u = 1; u < kCmFold; ++u) {
         zr[u].fill(!live[u], sizeof(Row) == 2 ? 0xff80u : 0xff800000u);
-        cr[u].fill(!live[u], 0u);
+        cr[u].fill(!live[u], sizeof(Row) == 2 ? 0x8000u : 0x80000000u);
       }
     }
     float v[kCmFold][8], c[kCmFold][8];
@@ -137,7 +138,11 @@ __device__ __forceinline__ void fold_tokens(PoolLane& st, const CompressArgs& a,
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[u][j] += br[u][j >> 2][j & 3];
     }
-    pool_fold<kCmFold>(st, v, c);
+    if constexpr (kSerial) {
+      pool_fold_serial<kCmFold>(st, v, c);
+    } else {
+      pool_fold<kCmFold>(st, v, c);
+    }
   }
 }
 
@@ -266,7 +271,7 @@ __global__ __launch_bounds__(kCmThreads, sizeof(Row) == 2 ? 3 : 2) void k_compre
           st.acc[j] = sbase[2 * a.channels + j];
         }
       }
-      fold_tokens<Row>(st, a, b, first_new, e, max(first_new, e * a.m), min(L, (e + 1) * a.m), slice, kSlices, gsafe);
+      fold_tokens<Row, kSlices == 1>(st, a, b, first_new, e, max(first_new, e * a.m), min(L, (e + 1) * a.m), slice, kSlices, gsafe);
     }
     merge_slices<kSlices>(sm, st);
     if (active && slice == 0) {

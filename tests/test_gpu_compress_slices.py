@@ -49,3 +49,28 @@ def test_compress_infinite_scores(dev, m) -> None:
     live = ~torch.isnan(want)
     assert bool(((got - want).abs() <= bound)[live].all())
     assert bool(torch.isnan(got[1, 3])) and bool(torch.isnan(got[0, 4]))
+
+
+@pytest.mark.parametrize("m,fp8", [(4, True), (4, False), (8, True), (15, False)])
+def test_short_blocks_are_the_same_at_once_and_by_tokens(dev, m, fp8) -> None:
+    """Entries (their fp8 codes) and states of blocks of one slice do not depend
+    on how the tokens were split over calls."""
+    from saint_kv import ops
+    from saint_kv._lib import fp8_entry_bytes
+
+    g = torch.Generator().manual_seed(m)
+    b, t, ch = 2, 40 * m + m // 2, 576
+    c, z = (torch.randn(b, t, ch, generator=g).to(dev, torch.bfloat16) for _ in range(2))
+    bias = torch.randn(m, ch, generator=g).to(dev)
+    got = []
+    for step in (t, 1, m + 3):
+        pool = torch.zeros(b, 64, fp8_entry_bytes(ch) if fp8 else ch, device=dev,
+                           dtype=torch.uint8 if fp8 else torch.bfloat16)
+        state = torch.zeros(b, 3, ch, device=dev)
+        for lo in range(0, t, step):
+            hi = min(lo + step, t)
+            ops.compress_append(pool, _i32([[0], [1]], dev), state, c[:, lo:hi].contiguous(), z[:, lo:hi].contiguous(),
+                                bias, _i32([hi] * b, dev), hi - lo)
+        got.append((pool, state))
+    for pool, state in got[1:]:
+        assert torch.equal(pool.view(torch.uint8), got[0][0].view(torch.uint8)) and torch.equal(state, got[0][1])
