@@ -220,6 +220,24 @@ int skv_compress_append(void* pool, int64_t entry_bytes, int64_t block_size, int
                         const int32_t* seq_lens, const int32_t* n_new, int32_t n_new_uniform,
                         int64_t m, int64_t channels, int32_t format, int64_t batch, void* stream);
 
+/* The same for several streams (layers, or a layer's main and indexer stream) of
+ * one batch at once: streams whose c/z rows have one type share a launch. */
+typedef struct skv_compress_stream {
+  void* pool;
+  int64_t entry_bytes, block_size, n_pages;
+  const int32_t* block_table;
+  int64_t bt_stride;
+  float* tail_state;
+  const void* c_new;
+  const void* z_new;
+  int64_t in_seq_stride, in_row_stride, in_len;
+  const float* bias;
+  int64_t m, channels;
+  int32_t format, reserved;
+} skv_compress_stream;
+int skv_compress_append_streams(const skv_compress_stream* streams, int64_t n_streams, const int32_t* seq_lens,
+                                const int32_t* n_new, int32_t n_new_uniform, int64_t batch, void* stream);
+
 /* ---- FP8 quantize-on-write --------------------------------------------------
  * skv_paged_append for SKV_FMT_FP8 entries: bf16 source rows of `channels`
  * dims are quantized per 1x128 block on the way into the pool

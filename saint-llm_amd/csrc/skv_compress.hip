@@ -224,7 +224,8 @@ __device__ __forceinline__ void emit_entry(const PoolLane& st, const CompressArg
   store_entry_group(entry, out, grp, groups, a.format, a.fp8_main);
 }
 
-// grid: (workgroups over the blocks, batch, 128-channel blocks).  Blocks
+// One workgroup of a stream: workgroup bx of gx over the blocks of sequence b,
+// 128-channel block zb.  Blocks
 // [e0, e1) of a sequence complete in this call; block e0 continues from the
 // stored state when the call before left it incomplete, and the tokens of
 // block e1, when it stays incomplete, go to the state.  When one call does
@@ -232,10 +233,8 @@ __device__ __forceinline__ void emit_entry(const PoolLane& st, const CompressArg
 // after block e0 (which is its first), so that the state is read before it
 // is written.
 template <class Row, int kSlices>
-__global__ __launch_bounds__(kCmThreads, sizeof(Row) == 2 ? 3 : 2) void k_compress_append(CompressArgs a) {
-  __shared__ CompressSmem sm;
+__device__ __forceinline__ void compress_workgroup(CompressSmem& sm, const CompressArgs& a, int bx, int gx, int b, int zb) {
   constexpr int kEntries = kCmGroups / kSlices;  // per workgroup and turn
-  const int b = blockIdx.y;
   const int L = a.lens[b];
   const int n = a.n_new ? a.n_new[b] : a.n_uni;
   if (n <= 0 || n > L || n > a.in_len) return;
@@ -244,14 +243,14 @@ __global__ __launch_bounds__(kCmThreads, sizeof(Row) == 2 ? 3 : 2) void k_compre
   const int e1 = L / a.m;
   const bool resumes = first_new > e0 * a.m;  // block e0 has a stored state
   const bool leaves = L > e1 * a.m;           // block e1 leaves one
-  bool last_turn = blockIdx.x == 0 && resumes && leaves && e1 > e0;
+  bool last_turn = bx == 0 && resumes && leaves && e1 > e0;
   const int n_units = e1 - e0 + (leaves && !(resumes && e1 > e0) ? 1 : 0);
   const int groups = a.channels >> 3;
-  const int grp = blockIdx.z * kCmLanes + threadIdx.x % kCmLanes;
+  const int grp = zb * kCmLanes + threadIdx.x % kCmLanes;
   const int gsafe = min(grp, groups - 1);  // lanes past the channels read the last group and store nothing
   const int slot = threadIdx.x / kCmLanes / kSlices, slice = threadIdx.x / kCmLanes % kSlices;
   float* sbase = a.state + static_cast<int64_t>(b) * 3 * a.channels + gsafe * 8;
-  int unit0 = blockIdx.x * kEntries;
+  int unit0 = bx * kEntries;
   while (unit0 < n_units || last_turn) {
     const bool in_last = unit0 >= n_units;
     if (in_last) __syncthreads();  // block e0's lanes have read the state
@@ -287,14 +286,150 @@ __global__ __launch_bounds__(kCmThreads, sizeof(Row) == 2 ? 3 : 2) void k_compre
       }
     }
     if (in_last) break;
-    unit0 += gridDim.x * kEntries;
+    unit0 += gx * kEntries;
     if constexpr (kSlices == 16) __syncthreads();  // the LDS is written again
+  }
+}
+
+// The streams of one launch, their workgroups one after another: a stream of
+// short blocks or few channels leaves the device partly idle at its end and a small
+// one all along, and each call costs the host more than a small one takes.  Five
+// streams (three layers; 4 prompts of 6,700-8,192 tokens): 112 us in five launches,
+// 73 in one (3.1 TB/s).
+constexpr int kCmStreams = 16;
+
+struct CompressStreams {
+  CompressArgs s[kCmStreams];
+  int32_t first[kCmStreams];  // first workgroup
+  int32_t turns[kCmStreams];  // workgroups over a sequence's blocks
+  int32_t zblocks[kCmStreams];
+  int32_t slices[kCmStreams];
+  int32_t n, batch;
+};
+
+template <class Row>
+__global__ __launch_bounds__(kCmThreads, sizeof(Row) == 2 ? 3 : 2) void k_compress_append(CompressStreams cs) {
+  __shared__ CompressSmem sm;
+  int i = 0;
+  while (i + 1 < cs.n && static_cast<int>(blockIdx.x) >= cs.first[i + 1]) ++i;  // uniform
+  const CompressArgs& a = cs.s[i];
+  const int l = blockIdx.x - cs.first[i];
+  const int rest = l / cs.zblocks[i], zb = l - rest * cs.zblocks[i];
+  const int b = rest / cs.turns[i], bx = rest - b * cs.turns[i];
+  switch (cs.slices[i]) {  // uniform
+    case 1: compress_workgroup<Row, 1>(sm, a, bx, cs.turns[i], b, zb); break;
+    case 4: compress_workgroup<Row, 4>(sm, a, bx, cs.turns[i], b, zb); break;
+    default: compress_workgroup<Row, 16>(sm, a, bx, cs.turns[i], b, zb); break;
   }
 }
 
 }  // namespace skv
 
 using namespace skv;
+
+// One stream's arguments, checked; 0 or an error code.
+static int compress_args(const char* what, const skv_compress_stream& x, int64_t batch, CompressArgs& a, bool& in_f32) {
+  in_f32 = (x.format & SKV_FMT_IN_F32) || (x.format & ~SKV_FMT_IN_F32) == SKV_FMT_F32;
+  const int32_t format = x.format & ~SKV_FMT_IN_F32;
+  const int64_t m = x.m, channels = x.channels;
+  if (m <= 0 || m > 4096) return set_error(SKV_EINVAL, "%s: compression_rate must be in [1, 4096]; got %lld", what, (long long)m);
+  if (channels <= 0 || (channels & 7) || channels > kPoolWave * 8 * kMaxGroups) {
+    return set_error(SKV_EINVAL, "%s: channels must be a multiple of 8 in [8, %d]; got %lld", what,
+                     kPoolWave * 8 * kMaxGroups, (long long)channels);
+  }
+  if (x.block_size <= 0 || x.bt_stride <= 0 || batch < 0 || batch > 65535) {
+    return set_error(SKV_EINVAL, "%s: bad block_size/bt_stride/batch", what);
+  }
+  const int fp8_main = (format == SKV_FMT_F32) ? ((x.entry_bytes == channels * 4) ? 0 : -1)
+                                               : entry_layout(format, channels, x.entry_bytes);
+  if (fp8_main < 0) {
+    return set_error(SKV_EINVAL,
+                     "%s: entry_bytes %lld does not match format %d with %lld channels (bf16: 2*channels; "
+                     "fp32: 4*channels; fp8: channels = 128*q + %d, entry_bytes = %lld)",
+                     what, (long long)x.entry_bytes, format, (long long)channels, SKV_FP8_ROPE_DIMS,
+                     (long long)SKV_FP8_ENTRY_BYTES(channels));
+  }
+  const uintptr_t align = reinterpret_cast<uintptr_t>(x.pool) | reinterpret_cast<uintptr_t>(x.tail_state) |
+                          reinterpret_cast<uintptr_t>(x.c_new) |
+                          reinterpret_cast<uintptr_t>(x.z_new) | static_cast<uintptr_t>(x.in_seq_stride) |
+                          static_cast<uintptr_t>(x.in_row_stride);
+  if (align & 15) return set_error(SKV_EINVAL, "%s: pointers and strides must be 16-byte aligned", what);
+  if (!x.bias || (reinterpret_cast<uintptr_t>(x.bias) & 3)) return set_error(SKV_EINVAL, "%s: bias must be fp32", what);
+  a = CompressArgs{};
+  a.pool = static_cast<uint8_t*>(x.pool);
+  a.entry_bytes = x.entry_bytes;
+  a.bs = static_cast<int>(x.block_size);
+  a.n_pages = x.n_pages;
+  a.bt = x.block_table;
+  a.bt_stride = x.bt_stride;
+  a.state = x.tail_state;
+  a.c_new = static_cast<const uint8_t*>(x.c_new);
+  a.z_new = static_cast<const uint8_t*>(x.z_new);
+  a.in_seq_stride = x.in_seq_stride;
+  a.in_row_stride = x.in_row_stride;
+  a.in_len = x.in_len;
+  a.bias = x.bias;
+  a.m = static_cast<int>(m);
+  a.channels = static_cast<int>(channels);
+  a.format = format;
+  a.fp8_main = fp8_main;
+  return SKV_OK;
+}
+
+static int launch_streams(const char* what, CompressStreams& cs, int64_t blocks, bool in_f32, void* stream) {
+  if (cs.n == 0) return SKV_OK;
+  const dim3 grid(static_cast<unsigned>(blocks));
+  if (in_f32) {
+    hipLaunchKernelGGL(k_compress_append<float>, grid, dim3(kCmThreads), 0, static_cast<hipStream_t>(stream), cs);
+  } else {
+    hipLaunchKernelGGL(k_compress_append<uint16_t>, grid, dim3(kCmThreads), 0, static_cast<hipStream_t>(stream), cs);
+  }
+  cs.n = 0;
+  return check_launch(what);
+}
+
+static int compress_streams(const char* what, const skv_compress_stream* streams, int64_t n_streams,
+                            const int32_t* seq_lens, const int32_t* n_new, int32_t n_new_uniform, int64_t batch,
+                            void* stream) {
+  CompressArgs a;
+  bool f32 = false, run_f32 = false;
+  for (int64_t i = 0; i < n_streams; ++i) {  // every stream before any launch
+    if (const int rc = compress_args(what, streams[i], batch, a, f32)) return rc;
+  }
+  if (!n_new && n_new_uniform < 0) return set_error(SKV_EINVAL, "%s: n_new_uniform must be >= 0", what);
+  if (batch == 0) return SKV_OK;
+  CompressStreams cs{};
+  cs.batch = static_cast<int32_t>(batch);
+  int64_t blocks = 0;
+  for (int64_t i = 0; i < n_streams; ++i) {
+    if (streams[i].in_len <= 0) continue;
+    if (const int rc = compress_args(what, streams[i], batch, a, f32)) return rc;
+    a.lens = seq_lens;
+    a.n_new = n_new;
+    a.n_uni = n_new_uniform;
+    if (cs.n == kCmStreams || (cs.n > 0 && f32 != run_f32)) {
+      if (const int rc = launch_streams(what, cs, blocks, run_f32, stream)) return rc;
+    }
+    if (cs.n == 0) blocks = 0;
+    run_f32 = f32;
+    // slices of an entry: at least 4 tokens per lane, which a turn of fold_tokens takes at once
+    // (blocks of 8 over 4 slices: 54 us for 4 x 8192 tokens of 576 channels, over one: 24 us)
+    const int slices = a.m < 16 ? 1 : a.m < 64 ? 4 : 16;
+    const int64_t zblocks = ceil_div(a.channels, 8 * kCmLanes);
+    // a call's tokens lie in at most ceil(in_len / m) + 1 blocks; past 2^26
+    // workgroups of a stream each takes several turns
+    const int64_t turns = std::min<int64_t>(ceil_div(ceil_div(a.in_len, a.m) + 1, kCmGroups / slices),
+                                            std::max<int64_t>(1, (1 << 26) / (batch * zblocks)));
+    cs.s[cs.n] = a;
+    cs.first[cs.n] = static_cast<int32_t>(blocks);
+    cs.turns[cs.n] = static_cast<int32_t>(turns);
+    cs.zblocks[cs.n] = static_cast<int32_t>(zblocks);
+    cs.slices[cs.n] = slices;
+    ++cs.n;
+    blocks += turns * batch * zblocks;
+  }
+  return launch_streams(what, cs, blocks, run_f32, stream);
+}
 
 extern "C" int skv_compress_append(void* pool, int64_t entry_bytes, int64_t block_size,
                                    int64_t n_pages, const int32_t* block_table, int64_t bt_stride,
@@ -303,71 +438,15 @@ extern "C" int skv_compress_append(void* pool, int64_t entry_bytes, int64_t bloc
                                    const float* bias, const int32_t* seq_lens, const int32_t* n_new,
                                    int32_t n_new_uniform, int64_t m, int64_t channels,
                                    int32_t format, int64_t batch, void* stream) {
-  const char* what = "skv_compress_append";
-  const bool in_f32 = (format & SKV_FMT_IN_F32) || (format & ~SKV_FMT_IN_F32) == SKV_FMT_F32;
-  format &= ~SKV_FMT_IN_F32;
-  if (m <= 0 || m > 4096) return set_error(SKV_EINVAL, "%s: compression_rate must be in [1, 4096]; got %lld", what, (long long)m);
-  if (channels <= 0 || (channels & 7) || channels > kPoolWave * 8 * kMaxGroups) {
-    return set_error(SKV_EINVAL, "%s: channels must be a multiple of 8 in [8, %d]; got %lld", what,
-                     kPoolWave * 8 * kMaxGroups, (long long)channels);
-  }
-  if (block_size <= 0 || bt_stride <= 0 || batch < 0 || batch > 65535) {
-    return set_error(SKV_EINVAL, "%s: bad block_size/bt_stride/batch", what);
-  }
-  const int fp8_main = (format == SKV_FMT_F32) ? ((entry_bytes == channels * 4) ? 0 : -1)
-                                               : entry_layout(format, channels, entry_bytes);
-  if (fp8_main < 0) {
-    return set_error(SKV_EINVAL,
-                     "%s: entry_bytes %lld does not match format %d with %lld channels (bf16: 2*channels; "
-                     "fp32: 4*channels; fp8: channels = 128*q + %d, entry_bytes = %lld)",
-                     what, (long long)entry_bytes, format, (long long)channels, SKV_FP8_ROPE_DIMS,
-                     (long long)SKV_FP8_ENTRY_BYTES(channels));
-  }
-  const uintptr_t align = reinterpret_cast<uintptr_t>(pool) | reinterpret_cast<uintptr_t>(tail_state) |
-                          reinterpret_cast<uintptr_t>(c_new) |
-                          reinterpret_cast<uintptr_t>(z_new) | static_cast<uintptr_t>(in_seq_stride) |
-                          static_cast<uintptr_t>(in_row_stride);
-  if (align & 15) return set_error(SKV_EINVAL, "%s: pointers and strides must be 16-byte aligned", what);
-  if (!bias || (reinterpret_cast<uintptr_t>(bias) & 3)) return set_error(SKV_EINVAL, "%s: bias must be fp32", what);
-  if (!n_new && n_new_uniform < 0) return set_error(SKV_EINVAL, "%s: n_new_uniform must be >= 0", what);
-  if (batch == 0 || in_len <= 0) return SKV_OK;
-  CompressArgs a{};
-  a.pool = static_cast<uint8_t*>(pool);
-  a.entry_bytes = entry_bytes;
-  a.bs = static_cast<int>(block_size);
-  a.n_pages = n_pages;
-  a.bt = block_table;
-  a.bt_stride = bt_stride;
-  a.state = tail_state;
-  a.c_new = static_cast<const uint8_t*>(c_new);
-  a.z_new = static_cast<const uint8_t*>(z_new);
-  a.in_seq_stride = in_seq_stride;
-  a.in_row_stride = in_row_stride;
-  a.in_len = in_len;
-  a.bias = bias;
-  a.lens = seq_lens;
-  a.n_new = n_new;
-  a.n_uni = n_new_uniform;
-  a.m = static_cast<int>(m);
-  a.channels = static_cast<int>(channels);
-  a.format = format;
-  a.fp8_main = fp8_main;
-  // slices of an entry: at least 4 tokens per lane, which a turn of fold_tokens takes at once
-  // (blocks of 8 over 4 slices: 54 us for 4 x 8192 tokens of 576 channels, over one: 24 us)
-  const int slices = m < 16 ? 1 : m < 64 ? 4 : 16;
-  // a call's tokens lie in at most ceil(in_len / m) + 1 blocks; past 2^20 workgroups each takes several turns
-  const int64_t turns = ceil_div(ceil_div(in_len, m) + 1, kCmGroups / slices);
-  const dim3 grid(static_cast<unsigned>(std::min<int64_t>(turns, 1 << 20)), static_cast<unsigned>(batch),
-                  static_cast<unsigned>(ceil_div(channels, 8 * kCmLanes)));
-  const auto launch = [&](auto kernel) {
-    hipLaunchKernelGGL(kernel, grid, dim3(kCmThreads), 0, static_cast<hipStream_t>(stream), a);
-  };
-  if (in_f32) {
-    slices == 1 ? launch(k_compress_append<float, 1>)
-                : slices == 4 ? launch(k_compress_append<float, 4>) : launch(k_compress_append<float, 16>);
-  } else {
-    slices == 1 ? launch(k_compress_append<uint16_t, 1>)
-                : slices == 4 ? launch(k_compress_append<uint16_t, 4>) : launch(k_compress_append<uint16_t, 16>);
-  }
-  return check_launch(what);
+  const skv_compress_stream x{pool,  entry_bytes,   block_size,    n_pages, block_table, bt_stride, tail_state, c_new,
+                              z_new, in_seq_stride, in_row_stride, in_len,  bias,        m,         channels,   format, 0};
+  return compress_streams("skv_compress_append", &x, 1, seq_lens, n_new, n_new_uniform, batch, stream);
+}
+
+extern "C" int skv_compress_append_streams(const skv_compress_stream* streams, int64_t n_streams,
+                                           const int32_t* seq_lens, const int32_t* n_new, int32_t n_new_uniform,
+                                           int64_t batch, void* stream) {
+  const char* what = "skv_compress_append_streams";
+  if (n_streams < 0 || (n_streams > 0 && !streams)) return set_error(SKV_EINVAL, "%s: no streams", what);
+  return compress_streams(what, streams, n_streams, seq_lens, n_new, n_new_uniform, batch, stream);
 }

@@ -64,6 +64,7 @@ SIGNATURES: dict[str, list] = {
         _P, _I64, _I64, _I64, _P, _I64, _P, _P, _P, _I64, _I64, _I64, _P, _P, _P, _I32, _I64, _I64,
         _I32, _I64, _P,
     ],
+    "skv_compress_append_streams": [_P, _I64, _P, _P, _I32, _I64, _P],
     "skv_fp8_quant_append": [
         _P, _I64, _I64, _I64, _P, _I64, _P, _P, _I32, _P, _I64, _I64, _I64, _I64, _I64, _P,
     ],
@@ -106,6 +107,17 @@ class PoolRef(ctypes.Structure):
     """skv_pool_ref: one pool sharing a block table."""
 
     _fields_ = [("base", ctypes.c_void_p), ("page_bytes", ctypes.c_int64)]
+
+class CompressStream(ctypes.Structure):
+    """skv_compress_stream: one stream of skv_compress_append_streams."""
+
+    _fields_ = [
+        ("pool", _P), ("entry_bytes", _I64), ("block_size", _I64), ("n_pages", _I64), ("block_table", _P),
+        ("bt_stride", _I64), ("tail_state", _P), ("c_new", _P), ("z_new", _P), ("in_seq_stride", _I64),
+        ("in_row_stride", _I64), ("in_len", _I64), ("bias", _P), ("m", _I64), ("channels", _I64),
+        ("format", _I32), ("reserved", _I32),
+    ]
+
 
 # entry points returning a size rather than a status code
 INT64_RESULTS = {"skv_topk_workspace_words", "skv_attention_workspace", "skv_attention_desc_size",

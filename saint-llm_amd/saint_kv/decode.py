@@ -442,11 +442,9 @@ class DecodeCache:
         lens_t = torch.as_tensor(lens.astype(np.int32), device=dev)
         self.reserve_entries(slice(None), [torch.as_tensor((lens // g.m).astype(np.int32), device=dev)
                                            for g in self.groups])
+        folds = []  # data's streams, folded together
         for i, spec in enumerate(self.layers):
-            if data is not None:
-                src = data[i]["kv"]
-                ops.ring_append(self.ring[i], lens_t, src, lens_t)
-            else:
+            if data is None:
                 self.ring[i].normal_(generator=generator)
             if spec.kind == "swa":
                 continue
@@ -457,8 +455,7 @@ class DecodeCache:
                                 self.c_indexer))
             for pool, state, bias, kc, kz, ch in streams:
                 if data is not None:
-                    ops.compress_append(pool, g.block_table, state, data[i][kc], data[i][kz], bias,
-                                        lens_t, lens_t)
+                    folds.append((pool, g.block_table, state, data[i][kc], data[i][kz], bias))
                     continue
                 self._fill_entries(pool, g, lens // spec.m, ch, generator, outlier_frac,
                                    outlier_scale)
@@ -472,6 +469,12 @@ class DecodeCache:
                         z = torch.randn(self.batch, t, ch, generator=generator, device=dev).to(torch.bfloat16)
                     ops.compress_append(pool, g.block_table, state, c, z, bias, lens_t,
                                         torch.as_tensor(tail.astype(np.int32), device=dev))
+        # one launch for all streams, issued before the rings' rows so that those
+        # calls' host work runs beside it
+        ops.compress_append_streams(folds, lens_t, lens_t)
+        if data is not None:
+            for i in range(len(self.layers)):
+                ops.ring_append(self.ring[i], lens_t, data[i]["kv"], lens_t)
         self.tok_lens.copy_(lens_t)
         self.host_lens = lens.copy()
 

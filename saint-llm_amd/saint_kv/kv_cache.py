@@ -350,6 +350,7 @@ class _CompressedLayer:
         the stream's token count after them.  Completed blocks go to the
         stream's pages (skv_compress_append) and its gather buffer."""
         lens = torch.full((self.batch_size,), tok_after, dtype=torch.int32, device=self.h_buffer.device)
+        folds = []
         for stream, state, (w_kv, w_z, bias) in zip(self._streams, self._tails, fast, strict=True):
             if n_complete > 0:
                 ops.reserve(stream.free_stack, stream.free_top, stream.block_table, stream.lens, n_complete,
@@ -364,9 +365,11 @@ class _CompressedLayer:
                         else torch.float32
                     c = w_kv(hh).to(pdt).contiguous()
                     z = w_z(hh).to(pdt).contiguous()
-                ops.compress_append(stream.pool, stream.block_table, state, c, z,
-                                    bias.detach().to(torch.float32).contiguous(), lens, n_fold)
-            if n_complete > 0:
+                folds.append((stream.pool, stream.block_table, state, c, z,
+                              bias.detach().to(torch.float32).contiguous()))
+        ops.compress_append_streams(folds, lens, n_fold)
+        if n_complete > 0:
+            for stream in self._streams:
                 first_page = stream.length // stream.block_size  # the page of the first new entry
                 stream.length += n_complete
                 ops.paged_gather(stream.pool, stream.block_table, stream.lens, stream._out,

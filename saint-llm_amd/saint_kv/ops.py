@@ -384,6 +384,12 @@ def compress_append(pool: torch.Tensor, block_table: torch.Tensor, tail_state: t
     and the entry is rounded once); ``bias`` fp32 [m, C] (m = compression
     rate).  Returns the entry format used.
     """
+    return compress_append_streams([(pool, block_table, tail_state, c_new, z_new, bias)], seq_lens, n_new)[0]
+
+
+def _compress_stream(pool: torch.Tensor, block_table: torch.Tensor, tail_state: torch.Tensor, c_new: torch.Tensor,
+                     z_new: torch.Tensor, bias: torch.Tensor, seq_lens: torch.Tensor) -> tuple:
+    """The checked skv_compress_stream fields of one stream."""
     n_pages, bs, rb = _check_pool(pool)
     _require_i32(block_table, "block_table")
     batch, bt_stride = block_table.shape
@@ -411,15 +417,24 @@ def compress_append(pool: torch.Tensor, block_table: torch.Tensor, tail_state: t
     if bias.dtype != torch.float32 or bias.dim() != 2 or bias.shape[1] != channels \
             or not bias.is_contiguous():
         raise ValueError(f"bias must be contiguous fp32 [m, {channels}]")
-    m = bias.shape[0]
-    n_ptr, n_uni = _n_new_args(n_new, batch)
     es = c_new.element_size()
-    _lib.call("skv_compress_append", pool.data_ptr(), rb, bs, n_pages, block_table.data_ptr(),
-              bt_stride, tail_state.data_ptr(), c_new.data_ptr(), z_new.data_ptr(),
-              c_new.stride(0) * es, c_new.stride(1) * es, c_new.shape[1], bias.data_ptr(),
-              seq_lens.data_ptr(), n_ptr, n_uni, m, channels, fmt | in_flag, batch,
-              _lib.stream_handle(pool.device))
-    return fmt
+    return (pool.data_ptr(), rb, bs, n_pages, block_table.data_ptr(), bt_stride, tail_state.data_ptr(),
+            c_new.data_ptr(), z_new.data_ptr(), c_new.stride(0) * es, c_new.stride(1) * es, c_new.shape[1],
+            bias.data_ptr(), bias.shape[0], channels, fmt | in_flag, 0)
+
+
+def compress_append_streams(streams: list[tuple], seq_lens: torch.Tensor, n_new: int | torch.Tensor) -> list[int]:
+    """``compress_append`` of several streams of one batch (layers, or a layer's
+    main and indexer stream) in one launch: ``streams`` holds (pool, block_table,
+    tail_state, c_new, z_new, bias) each.  Returns the entry formats used."""
+    if not streams:
+        return []
+    arr = (_lib.CompressStream * len(streams))(*[_compress_stream(*s, seq_lens) for s in streams])
+    batch = seq_lens.shape[0]
+    n_ptr, n_uni = _n_new_args(n_new, batch)
+    _lib.call("skv_compress_append_streams", arr, len(streams), seq_lens.data_ptr(), n_ptr, n_uni, batch,
+              _lib.stream_handle(seq_lens.device))
+    return [x.format & ~_lib.SKV_FMT_IN_F32 for x in arr]
 
 
 def fp8_quant_append(pool: torch.Tensor, block_table: torch.Tensor, seq_lens: torch.Tensor,
