@@ -439,9 +439,10 @@ class DecodeCache:
         if (self.host_lens != 0).any():
             raise RuntimeError("prefill needs empty sequences")
         dev = self.device
-        lens_t = torch.as_tensor(lens.astype(np.int32), device=dev)
-        self.reserve_entries(slice(None), [torch.as_tensor((lens // g.m).astype(np.int32), device=dev)
-                                           for g in self.groups])
+        # the token counts and every group's entry counts in one copy to the device
+        counts = torch.as_tensor(np.stack([lens, *(lens // g.m for g in self.groups)]).astype(np.int32), device=dev)
+        lens_t = counts[0]
+        self.reserve_entries(slice(None), list(counts[1:]))
         folds = []  # data's streams, folded together
         for i, spec in enumerate(self.layers):
             if data is None:

@@ -20,7 +20,7 @@ INT32 = torch.int32
 def _require_gpu(t: torch.Tensor, name: str) -> None:
     if not isinstance(t, torch.Tensor):
         raise TypeError(f"{name} must be a torch.Tensor")
-    if t.device.type != "cuda":
+    if not t.is_cuda:
         raise RuntimeError(
             f"{name} is on {t.device}; saint_kv runs only on a ROCm GPU (no CPU fallback)",
         )
