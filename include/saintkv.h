@@ -113,6 +113,14 @@ int skv_paged_gather(void* dst, const int64_t* dst_row_offsets, int64_t dst_seq_
                      int64_t block_size, int64_t n_pages, const int32_t* block_table,
                      int64_t bt_stride, const int32_t* seq_lens, int64_t batch, void* stream);
 
+/* skv_paged_gather of the rows from page first_page (< bt_stride) of every
+ * sequence on; the dst rows before are left as they are. */
+int skv_paged_gather_from(void* dst, const int64_t* dst_row_offsets, int64_t dst_seq_stride_rows,
+                          int64_t dst_capacity_rows, const void* pool, int64_t row_bytes,
+                          int64_t block_size, int64_t n_pages, const int32_t* block_table,
+                          int64_t bt_stride, const int32_t* seq_lens, int64_t first_page, int64_t batch,
+                          void* stream);
+
 /* skv_append_gather: skv_paged_append + skv_paged_gather in one launch; new
  * rows go from src to both the pool and dst.  One decode step of
  * SWAKVCacheLayer.append (kv_cache.py:63-83) on paged storage. */
@@ -122,6 +130,16 @@ int skv_append_gather(void* dst, const int64_t* dst_row_offsets, int64_t dst_seq
                       int64_t bt_stride, const int32_t* seq_lens, const int32_t* n_new,
                       int32_t n_new_uniform, const void* src, int64_t src_seq_stride,
                       int64_t src_row_stride, int64_t src_len, int64_t batch, void* stream);
+
+/* skv_append_gather from page first_page (< bt_stride) of every sequence on; the
+ * new rows must lie there. */
+int skv_append_gather_from(void* dst, const int64_t* dst_row_offsets, int64_t dst_seq_stride_rows,
+                           int64_t dst_capacity_rows, void* pool, int64_t row_bytes,
+                           int64_t block_size, int64_t n_pages, const int32_t* block_table,
+                           int64_t bt_stride, const int32_t* seq_lens, const int32_t* n_new,
+                           int32_t n_new_uniform, const void* src, int64_t src_seq_stride,
+                           int64_t src_row_stride, int64_t src_len, int64_t first_page, int64_t batch,
+                           void* stream);
 
 /* skv_decode_append_gather: skv_reserve + skv_append_gather as one decode
  * step in two launches, the copy cut into 4 KB slices of page units (one

@@ -124,6 +124,9 @@ struct CopyArgs {
   int64_t src_row_stride;
   int64_t src_len;  // rows per sequence available in src
   int batch;
+  // gathers: page of every sequence that the copy starts at (lengths shifted by
+  // the caller took two launches more: 15% of a tiny model's drop-in layers)
+  int first_page;
 };
 
 // Copy `nchunks` 16-byte chunks; kCopyUnroll loads in flight per lane.
@@ -192,7 +195,8 @@ __global__ __launch_bounds__(kCopyThreads) void k_paged_copy(CopyArgs a) {
         const int n = a.n_new ? a.n_new[b] : a.n_uni;
         units = (n + kAppendRowsPerUnit - 1) / kAppendRowsPerUnit;
       } else {
-        units = (L + a.bs - 1) / a.bs;
+        // pages from the first one on that the table can hold
+        units = max(static_cast<int>(min<int64_t>((L + a.bs - 1) / a.bs, a.bt_stride)) - a.first_page, 0);
       }
     }
     int tot;
@@ -226,9 +230,10 @@ __global__ __launch_bounds__(kCopyThreads) void k_paged_copy(CopyArgs a) {
       }
       continue;
     }
-    const int r0 = k * a.bs;
+    const int p = a.first_page + k;
+    const int r0 = p * a.bs;
     const int r1 = min(L, r0 + a.bs);
-    const int32_t page = (k < a.bt_stride) ? a.bt[static_cast<int64_t>(b) * a.bt_stride + k] : -1;
+    const int32_t page = a.bt[static_cast<int64_t>(b) * a.bt_stride + p];  // p < bt_stride
     if (page < 0 || page >= a.n_pages) continue;  // unmapped: skipped, never dereferenced
     uint8_t* page_base = a.pool + static_cast<int64_t>(page) * page_bytes;
     const int64_t drow0 = a.dst_off ? a.dst_off[b] : static_cast<int64_t>(b) * a.dst_stride_rows;
@@ -286,8 +291,11 @@ template <int kMode>
 static int launch_copy(const CopyArgs& a, hipStream_t stream, const char* what) {
   if (a.batch == 0) return SKV_OK;
   const size_t shmem = (a.batch + 1 + 17) * sizeof(int);
-  hipLaunchKernelGGL(k_paged_copy<kMode>, dim3(kPersistentBlocks), dim3(kCopyThreads), shmem,
-                     stream, a);
+  // a gather has at most a unit per page from the first one on (a small cache's
+  // 2,048 workgroups, nearly all idle, took 4.2 us)
+  const int64_t units = kMode == 1 ? kPersistentBlocks : a.batch * (a.bt_stride - a.first_page);
+  const dim3 grid(static_cast<unsigned>(units < kPersistentBlocks ? units : kPersistentBlocks));
+  hipLaunchKernelGGL(k_paged_copy<kMode>, grid, dim3(kCopyThreads), shmem, stream, a);
   return check_launch(what);
 }
 
@@ -559,13 +567,17 @@ extern "C" int skv_paged_append(void* pool, int64_t row_bytes, int64_t block_siz
   return launch_copy<1>(a, static_cast<hipStream_t>(stream), "skv_paged_append");
 }
 
-extern "C" int skv_paged_gather(void* dst, const int64_t* dst_row_offsets,
+extern "C" int skv_paged_gather_from(void* dst, const int64_t* dst_row_offsets,
                                 int64_t dst_seq_stride_rows, int64_t dst_capacity_rows,
                                 const void* pool, int64_t row_bytes, int64_t block_size,
                                 int64_t n_pages, const int32_t* block_table, int64_t bt_stride,
-                                const int32_t* seq_lens, int64_t batch, void* stream) {
+                                const int32_t* seq_lens, int64_t first_page, int64_t batch,
+                                void* stream) {
   int rc = validate_copy("skv_paged_gather", row_bytes, block_size, batch, bt_stride, pool, dst);
   if (rc) return rc;
+  if (first_page < 0 || first_page >= bt_stride) {
+    return set_error(SKV_EINVAL, "skv_paged_gather: first_page must be in [0, bt_stride)");
+  }
   CopyArgs a{};
   a.dst = static_cast<uint8_t*>(dst);
   a.dst_off = dst_row_offsets;
@@ -579,19 +591,32 @@ extern "C" int skv_paged_gather(void* dst, const int64_t* dst_row_offsets,
   a.bt_stride = bt_stride;
   a.lens = seq_lens;
   a.batch = static_cast<int>(batch);
+  a.first_page = static_cast<int>(first_page);
   return launch_copy<0>(a, static_cast<hipStream_t>(stream), "skv_paged_gather");
 }
 
-extern "C" int skv_append_gather(void* dst, const int64_t* dst_row_offsets,
+extern "C" int skv_paged_gather(void* dst, const int64_t* dst_row_offsets,
+                                int64_t dst_seq_stride_rows, int64_t dst_capacity_rows,
+                                const void* pool, int64_t row_bytes, int64_t block_size,
+                                int64_t n_pages, const int32_t* block_table, int64_t bt_stride,
+                                const int32_t* seq_lens, int64_t batch, void* stream) {
+  return skv_paged_gather_from(dst, dst_row_offsets, dst_seq_stride_rows, dst_capacity_rows, pool, row_bytes,
+                               block_size, n_pages, block_table, bt_stride, seq_lens, 0, batch, stream);
+}
+
+extern "C" int skv_append_gather_from(void* dst, const int64_t* dst_row_offsets,
                                  int64_t dst_seq_stride_rows, int64_t dst_capacity_rows, void* pool,
                                  int64_t row_bytes, int64_t block_size, int64_t n_pages,
                                  const int32_t* block_table, int64_t bt_stride,
                                  const int32_t* seq_lens, const int32_t* n_new,
                                  int32_t n_new_uniform, const void* src, int64_t src_seq_stride,
-                                 int64_t src_row_stride, int64_t src_len, int64_t batch,
-                                 void* stream) {
+                                 int64_t src_row_stride, int64_t src_len, int64_t first_page,
+                                 int64_t batch, void* stream) {
   int rc = validate_copy("skv_append_gather", row_bytes, block_size, batch, bt_stride, pool, dst);
   if (rc) return rc;
+  if (first_page < 0 || first_page >= bt_stride) {
+    return set_error(SKV_EINVAL, "skv_append_gather: first_page must be in [0, bt_stride)");
+  }
   if ((rc = validate_src("skv_append_gather", src, src_seq_stride, src_row_stride))) return rc;
   CopyArgs a{};
   a.dst = static_cast<uint8_t*>(dst);
@@ -612,7 +637,21 @@ extern "C" int skv_append_gather(void* dst, const int64_t* dst_row_offsets,
   a.src_row_stride = src_row_stride;
   a.src_len = src_len;
   a.batch = static_cast<int>(batch);
+  a.first_page = static_cast<int>(first_page);
   return launch_copy<2>(a, static_cast<hipStream_t>(stream), "skv_append_gather");
+}
+
+extern "C" int skv_append_gather(void* dst, const int64_t* dst_row_offsets,
+                                 int64_t dst_seq_stride_rows, int64_t dst_capacity_rows, void* pool,
+                                 int64_t row_bytes, int64_t block_size, int64_t n_pages,
+                                 const int32_t* block_table, int64_t bt_stride,
+                                 const int32_t* seq_lens, const int32_t* n_new,
+                                 int32_t n_new_uniform, const void* src, int64_t src_seq_stride,
+                                 int64_t src_row_stride, int64_t src_len, int64_t batch,
+                                 void* stream) {
+  return skv_append_gather_from(dst, dst_row_offsets, dst_seq_stride_rows, dst_capacity_rows, pool, row_bytes,
+                                block_size, n_pages, block_table, bt_stride, seq_lens, n_new, n_new_uniform, src,
+                                src_seq_stride, src_row_stride, src_len, 0, batch, stream);
 }
 
 extern "C" int skv_plan_units(int32_t* free_stack, int32_t* free_top, int64_t n_pages,

@@ -44,9 +44,14 @@ SIGNATURES: dict[str, list] = {
         _P, _I64, _I64, _I64, _P, _I64, _P, _P, _I32, _P, _I64, _I64, _I64, _I64, _P,
     ],
     "skv_paged_gather": [_P, _P, _I64, _I64, _P, _I64, _I64, _I64, _P, _I64, _P, _I64, _P],
+    "skv_paged_gather_from": [_P, _P, _I64, _I64, _P, _I64, _I64, _I64, _P, _I64, _P, _I64, _I64, _P],
     "skv_append_gather": [
         _P, _P, _I64, _I64, _P, _I64, _I64, _I64, _P, _I64, _P, _P, _I32, _P, _I64, _I64, _I64,
         _I64, _P,
+    ],
+    "skv_append_gather_from": [
+        _P, _P, _I64, _I64, _P, _I64, _I64, _I64, _P, _I64, _P, _P, _I32, _P, _I64, _I64, _I64,
+        _I64, _I64, _P,
     ],
     "skv_decode_append_gather": [
         _P, _P, _I64, _P, _I64, _P, _P, _I32, _P, _P, _P, _I64, _I64, _P, _I64, _I64, _P, _I64,

@@ -87,6 +87,7 @@ class _PagedRows:
         self.block_table = torch.full((batch, self.max_pages), -1, dtype=torch.int32, device=device)
         self.lens = torch.zeros(batch, dtype=torch.int32, device=device)
         self.status = torch.zeros(1, dtype=torch.int32, device=device)
+        self._all: Tensor | None = None  # reset's release mask, made by the first one
         self._out = torch.zeros(batch, max_rows, *store_shape, dtype=dtype, device=device)
         ops.free_stack_init(self.free_stack, self.free_top)
         self.length = 0
@@ -111,8 +112,9 @@ class _PagedRows:
 
     def reset(self) -> None:
         if self.length:
-            mask = torch.ones(self.batch, dtype=torch.uint8, device=self.pool.device)
-            ops.release(self.free_stack, self.free_top, self.block_table, self.lens, mask,
+            if self._all is None:
+                self._all = torch.ones(self.batch, dtype=torch.uint8, device=self.pool.device)
+            ops.release(self.free_stack, self.free_top, self.block_table, self.lens, self._all,
                         self.block_size, self.status)
         self.length = 0
 
