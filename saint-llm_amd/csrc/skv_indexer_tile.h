@@ -35,8 +35,6 @@ constexpr int kIdxQRow = 32 * kIdxMaxKS + 8;          // LDS row of a query head
 
 __device__ __forceinline__ bf16x8 as_bf16x8(u32x4 v) { return __builtin_bit_cast(bf16x8, v); }
 
-// The query row in LDS, heads padded to 64 and channels to 128 with zeros;
-// rows of 272 bytes put the 16 lanes that read one A operand on distinct banks.
 // A chunk of t_new query tokens per sequence scored against the n_blocks
 // contiguous keys of each sequence (key_rows rows apart), token t against those
 // below (offset + t) / m.  scores: [batch * t_new, n_blocks].
@@ -51,6 +49,8 @@ struct IndexerChunk {
 int indexer_check_query(const char* what, int64_t n_heads, int64_t channels);
 int launch_indexer_chunk(const IndexerChunk& x, hipStream_t s);
 
+// The query row in LDS, heads padded to 64 and channels to 128 with zeros;
+// rows of 272 bytes put the 16 lanes that read one A operand on distinct banks.
 struct IndexerSmem {
   alignas(16) uint16_t q[16 * kIdxMaxHB][kIdxQRow];
 };
