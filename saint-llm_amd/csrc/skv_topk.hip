@@ -296,7 +296,7 @@ extern "C" int skv_topk_select_decode(const float* scores, int64_t score_stride,
 // of a workgroup are not scored.  With the mask, the keys' copy and the picks'
 // widening in launches of their own a single token over 250 entries took 83 us,
 // bound by them; now 19.  2,048 tokens from position 15 on, 64 heads: 39 us (327
-// with all entries scored and the radix selection); from 14,336 on 171.
+// with all entries scored and the radix selection); from 14,336 on 147.
 extern "C" int skv_indexer_topk(const void* q, const float* w, const void* keys, int64_t key_rows, float* scores,
                                 int64_t* out_idx, int64_t batch, int64_t t_new, int64_t n_heads, int64_t channels,
                                 int64_t n_blocks, int64_t cache_offset, int64_t m, int64_t k, void* stream) {
