@@ -208,6 +208,17 @@ int skv_ring_append(void* ring, int64_t window, int64_t row_bytes, const int32_t
                     const int32_t* n_new, int32_t n_new_uniform, const void* src,
                     int64_t src_seq_stride, int64_t src_row_stride, int64_t src_len,
                     int64_t batch, void* stream);
+
+/* The same for the rings of several layers of one batch, up to 16 a launch. */
+typedef struct skv_ring_layer {
+  void* ring;
+  int64_t window, row_bytes;
+  const void* src;
+  int64_t src_seq_stride, src_row_stride, src_len;
+} skv_ring_layer;
+int skv_ring_append_layers(const skv_ring_layer* rings, int64_t n_rings, const int32_t* seq_lens,
+                           const int32_t* n_new, int32_t n_new_uniform, int64_t batch, void* stream);
+
 int skv_ring_read(void* dst, int64_t dst_seq_stride_rows, int64_t dst_capacity_rows,
                   const void* ring, int64_t window, int64_t row_bytes, const int32_t* seq_lens,
                   int64_t batch, void* stream);

@@ -28,8 +28,18 @@ struct RingArgs {
   int batch;
 };
 
-// grid: (ceil(W / rows), batch).  Row slot r of the ring of sequence b.
-__global__ __launch_bounds__(kRingThreads) void k_ring_append(RingArgs a) {
+// The rings of several layers in one launch: a prompt's were calls of 4-6 us of
+// copying and as much host work, one after another (4 prompts of 8k tokens through
+// three layers: 277 us the request with three calls, 267 with one).
+constexpr int kRingLayers = 16;
+
+struct RingLayers {
+  RingArgs r[kRingLayers];
+};
+
+// grid: (ceil(W / rows), batch, rings).  Row slot r of the ring of sequence b.
+__global__ __launch_bounds__(kRingThreads) void k_ring_append(RingLayers layers) {
+  const RingArgs& a = layers.r[blockIdx.z];
   const int b = blockIdx.y;
   const int L = a.lens[b];
   const int n = a.n_new ? a.n_new[b] : a.n_uni;
@@ -98,36 +108,58 @@ static int validate_ring(const char* what, int64_t window, int64_t row_bytes, in
 
 using namespace skv;
 
+static int ring_append_layers(const char* what, const skv_ring_layer* rings, int64_t n_rings, const int32_t* seq_lens,
+                              const int32_t* n_new, int32_t n_new_uniform, int64_t batch, void* stream) {
+  for (int64_t i = 0; i < n_rings; ++i) {  // every ring before any launch
+    const skv_ring_layer& x = rings[i];
+    if (const int rc = validate_ring(what, x.window, x.row_bytes, batch, x.ring)) return rc;
+    if (!x.src || (reinterpret_cast<uintptr_t>(x.src) & 15) || (x.src_seq_stride & 15) || (x.src_row_stride & 15)) {
+      return set_error(SKV_EINVAL, "%s: src pointer and strides must be 16-byte aligned", what);
+    }
+  }
+  if (!n_new && n_new_uniform < 0) return set_error(SKV_EINVAL, "%s: n_new_uniform must be >= 0", what);
+  if (batch == 0) return SKV_OK;
+  for (int64_t i0 = 0; i0 < n_rings; i0 += kRingLayers) {
+    RingLayers layers{};
+    const int64_t n = n_rings - i0 < kRingLayers ? n_rings - i0 : kRingLayers;
+    int64_t window = 0;
+    for (int64_t i = 0; i < n; ++i) {
+      const skv_ring_layer& x = rings[i0 + i];
+      RingArgs& a = layers.r[i];
+      a.ring = static_cast<uint8_t*>(x.ring);
+      a.window = x.window;
+      a.row_bytes = x.row_bytes;
+      a.lens = seq_lens;
+      a.n_new = n_new;
+      a.n_uni = n_new_uniform;
+      a.src = static_cast<const uint8_t*>(x.src);
+      a.src_seq_stride = x.src_seq_stride;
+      a.src_row_stride = x.src_row_stride;
+      a.src_len = x.src_len;
+      a.batch = static_cast<int>(batch);
+      window = x.window > window ? x.window : window;
+    }
+    const dim3 grid(static_cast<unsigned>(ceil_div(window, kRingRowsPerBlock)), static_cast<unsigned>(batch),
+                    static_cast<unsigned>(n));
+    hipLaunchKernelGGL(k_ring_append, grid, dim3(kRingThreads), 0, static_cast<hipStream_t>(stream), layers);
+    if (const int rc = check_launch(what)) return rc;
+  }
+  return SKV_OK;
+}
+
 extern "C" int skv_ring_append(void* ring, int64_t window, int64_t row_bytes,
                                const int32_t* seq_lens, const int32_t* n_new, int32_t n_new_uniform,
                                const void* src, int64_t src_seq_stride, int64_t src_row_stride,
                                int64_t src_len, int64_t batch, void* stream) {
-  int rc = validate_ring("skv_ring_append", window, row_bytes, batch, ring);
-  if (rc) return rc;
-  if (!src || (reinterpret_cast<uintptr_t>(src) & 15) || (src_seq_stride & 15) ||
-      (src_row_stride & 15)) {
-    return set_error(SKV_EINVAL, "skv_ring_append: src pointer and strides must be 16-byte aligned");
-  }
-  if (!n_new && n_new_uniform < 0) {
-    return set_error(SKV_EINVAL, "skv_ring_append: n_new_uniform must be >= 0");
-  }
-  if (batch == 0) return SKV_OK;
-  RingArgs a{};
-  a.ring = static_cast<uint8_t*>(ring);
-  a.window = window;
-  a.row_bytes = row_bytes;
-  a.lens = seq_lens;
-  a.n_new = n_new;
-  a.n_uni = n_new_uniform;
-  a.src = static_cast<const uint8_t*>(src);
-  a.src_seq_stride = src_seq_stride;
-  a.src_row_stride = src_row_stride;
-  a.src_len = src_len;
-  a.batch = static_cast<int>(batch);
-  const dim3 grid(static_cast<unsigned>(ceil_div(window, kRingRowsPerBlock)),
-                  static_cast<unsigned>(batch));
-  hipLaunchKernelGGL(k_ring_append, grid, dim3(kRingThreads), 0, static_cast<hipStream_t>(stream), a);
-  return check_launch("skv_ring_append");
+  const skv_ring_layer x{ring, window, row_bytes, src, src_seq_stride, src_row_stride, src_len};
+  return ring_append_layers("skv_ring_append", &x, 1, seq_lens, n_new, n_new_uniform, batch, stream);
+}
+
+extern "C" int skv_ring_append_layers(const skv_ring_layer* rings, int64_t n_rings, const int32_t* seq_lens,
+                                      const int32_t* n_new, int32_t n_new_uniform, int64_t batch, void* stream) {
+  const char* what = "skv_ring_append_layers";
+  if (n_rings < 0 || (n_rings > 0 && !rings)) return set_error(SKV_EINVAL, "%s: no rings", what);
+  return ring_append_layers(what, rings, n_rings, seq_lens, n_new, n_new_uniform, batch, stream);
 }
 
 extern "C" int skv_ring_read(void* dst, int64_t dst_seq_stride_rows, int64_t dst_capacity_rows,

@@ -64,6 +64,7 @@ SIGNATURES: dict[str, list] = {
     "skv_plan_units": [_P, _P, _I64, _P, _I64, _P, _P, _I32, _P, _P, _I64, _I64, _P, _I64, _I64, _P],
     "skv_copy_slices": [_P, _I64, _P, _I64, _I64, _I64, _P, _I64, _I64, _I64, _P, _I64, _P],
     "skv_ring_append": [_P, _I64, _I64, _P, _P, _I32, _P, _I64, _I64, _I64, _I64, _P],
+    "skv_ring_append_layers": [_P, _I64, _P, _P, _I32, _I64, _P],
     "skv_ring_read": [_P, _I64, _I64, _P, _I64, _I64, _P, _I64, _P],
     "skv_compress_append": [
         _P, _I64, _I64, _I64, _P, _I64, _P, _P, _P, _I64, _I64, _I64, _P, _P, _P, _I32, _I64, _I64,
@@ -121,6 +122,15 @@ class CompressStream(ctypes.Structure):
         ("bt_stride", _I64), ("tail_state", _P), ("c_new", _P), ("z_new", _P), ("in_seq_stride", _I64),
         ("in_row_stride", _I64), ("in_len", _I64), ("bias", _P), ("m", _I64), ("channels", _I64),
         ("format", _I32), ("reserved", _I32),
+    ]
+
+
+class RingLayer(ctypes.Structure):
+    """skv_ring_layer: one ring of skv_ring_append_layers."""
+
+    _fields_ = [
+        ("ring", _P), ("window", _I64), ("row_bytes", _I64), ("src", _P), ("src_seq_stride", _I64),
+        ("src_row_stride", _I64), ("src_len", _I64),
     ]
 
 

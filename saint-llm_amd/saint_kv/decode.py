@@ -470,12 +470,11 @@ class DecodeCache:
                         z = torch.randn(self.batch, t, ch, generator=generator, device=dev).to(torch.bfloat16)
                     ops.compress_append(pool, g.block_table, state, c, z, bias, lens_t,
                                         torch.as_tensor(tail.astype(np.int32), device=dev))
-        # one launch for all streams, issued before the rings' rows so that those
-        # calls' host work runs beside it
+        # one launch for all streams, issued before the rings' rows so that that
+        # call's host work runs beside it
         ops.compress_append_streams(folds, lens_t, lens_t)
         if data is not None:
-            for i in range(len(self.layers)):
-                ops.ring_append(self.ring[i], lens_t, data[i]["kv"], lens_t)
+            ops.ring_append_layers([(self.ring[i], data[i]["kv"]) for i in range(len(self.layers))], lens_t, lens_t)
         self.tok_lens.copy_(lens_t)
         self.host_lens = lens.copy()
 

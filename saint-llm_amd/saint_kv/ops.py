@@ -327,15 +327,26 @@ def _check_ring(ring: torch.Tensor) -> tuple[int, int, int]:
 def ring_append(ring: torch.Tensor, seq_lens: torch.Tensor, src: torch.Tensor,
                 n_new: int | torch.Tensor) -> None:
     """Write the newest ``n_new`` tokens (``seq_lens`` already counts them) into the ring."""
-    batch, window, rb = _check_ring(ring)
-    _require_i32(seq_lens, "seq_lens", (batch,))
-    _require_gpu(src, "src")
-    if src.shape[0] != batch:
-        raise ValueError(f"src batch {src.shape[0]} != ring batch {batch}")
-    s_seq, s_row = _row_view_strides(src, rb, "src")
+    ring_append_layers([(ring, src)], seq_lens, n_new)
+
+
+def ring_append_layers(rings: list[tuple], seq_lens: torch.Tensor, n_new: int | torch.Tensor) -> None:
+    """``ring_append`` of several layers of one batch in one launch: (ring, src) each."""
+    layers = []
+    for ring, src in rings:
+        batch, window, rb = _check_ring(ring)
+        _require_i32(seq_lens, "seq_lens", (batch,))
+        _require_gpu(src, "src")
+        if src.shape[0] != batch:
+            raise ValueError(f"src batch {src.shape[0]} != ring batch {batch}")
+        s_seq, s_row = _row_view_strides(src, rb, "src")
+        layers.append((ring.data_ptr(), window, rb, src.data_ptr(), s_seq, s_row, src.shape[1]))
+    if not layers:
+        return
+    batch = seq_lens.shape[0]
     n_ptr, n_uni = _n_new_args(n_new, batch)
-    _lib.call("skv_ring_append", ring.data_ptr(), window, rb, seq_lens.data_ptr(), n_ptr, n_uni,
-              src.data_ptr(), s_seq, s_row, src.shape[1], batch, _lib.stream_handle(ring.device))
+    _lib.call("skv_ring_append_layers", (_lib.RingLayer * len(layers))(*layers), len(layers), seq_lens.data_ptr(),
+              n_ptr, n_uni, batch, _lib.stream_handle(seq_lens.device))
 
 
 def ring_read(ring: torch.Tensor, seq_lens: torch.Tensor, out: torch.Tensor) -> torch.Tensor:
