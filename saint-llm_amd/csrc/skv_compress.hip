@@ -86,15 +86,6 @@ struct RawRow {
       for (int j = 0; j < 8; ++j) f[j] = __uint_as_float(v[j >> 2][j & 3]);
     }
   }
-  // every channel `bits` (the bits of a value of this type) where dead
-  __device__ __forceinline__ void fill(bool dead, uint32_t bits) {
-    const uint32_t word = kVecs == 1 ? bits | (bits << 16) : bits;
-#pragma unroll
-    for (int i = 0; i < kVecs; ++i) {
-#pragma unroll
-      for (int q = 0; q < 4; ++q) v[i][q] = dead ? word : v[i][q];
-    }
-  }
 };
 
 // Tokens first + slice + stride * i < p1 of entry e (sequence b) folded into
@@ -123,13 +114,6 @@ __device__ __forceinline__ void fold_tokens(PoolLane& st, const CompressArgs& a,
       br[u][1] = bp[1];
     }
     __builtin_amdgcn_sched_barrier(0);
-    if (__ballot(!live[kCmFold - 1])) {  // tokens past the end: value -inf, row -0: nothing is added
-#pragma unroll
-      for (int u = 1; u < kCmFold; ++u) {
-        zr[u].fill(!live[u], sizeof(Row) == 2 ? 0xff80u : 0xff800000u);
-        cr[u].fill(!live[u], sizeof(Row) == 2 ? 0x8000u : 0x80000000u);
-      }
-    }
     float v[kCmFold][8], c[kCmFold][8];
 #pragma unroll
     for (int u = 0; u < kCmFold; ++u) {
@@ -138,9 +122,27 @@ __device__ __forceinline__ void fold_tokens(PoolLane& st, const CompressArgs& a,
 #pragma unroll
       for (int j = 0; j < 8; ++j) v[u][j] += br[u][j >> 2][j & 3];
     }
+    const bool part = __ballot(!live[kCmFold - 1]);  // a turn past some lane's last token
     if constexpr (kSerial) {
-      pool_fold_serial<kCmFold>(st, v, c);
+      if (part) {
+#pragma unroll
+        for (int u = 0; u < kCmFold; ++u) {
+          if (live[u]) pool_fold_token(st, v[u], c[u]);
+        }
+      } else {
+        pool_fold_serial<kCmFold>(st, v, c);
+      }
     } else {
+      if (part) {  // tokens past the end: value -inf whatever the bias, row -0: nothing is added
+#pragma unroll
+        for (int u = 1; u < kCmFold; ++u) {
+#pragma unroll
+          for (int j = 0; j < 8; ++j) {
+            v[u][j] = live[u] ? v[u][j] : -INFINITY;
+            c[u][j] = live[u] ? c[u][j] : -0.f;
+          }
+        }
+      }
       pool_fold<kCmFold>(st, v, c);
     }
   }

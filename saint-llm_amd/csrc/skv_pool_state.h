@@ -63,23 +63,27 @@ __device__ __forceinline__ void pool_fold(PoolLane& st, const float (&v)[N][8], 
   }
 }
 
-// Folds one token after another, as the decode step does: the same sums whether a
+// Folds one token (values v, rows c).  Where v - max is NaN the weight is 1, as in
+// pool_weight.
+__device__ __forceinline__ void pool_fold_token(PoolLane& st, const float (&v)[8], const float (&c)[8]) {
+#pragma unroll
+  for (int j = 0; j < 8; ++j) {
+    const float d = v[j] - st.mx[j];
+    const bool up = v[j] > st.mx[j];
+    const float t = d != d ? 1.f : expf(-__builtin_fabsf(d));  // rescales the state, or weighs the token
+    st.sum[j] = fmaf(t, up ? st.sum[j] : 1.f, up ? 1.f : st.sum[j]);
+    st.acc[j] = fmaf(t, up ? st.acc[j] : c[j], up ? c[j] : st.acc[j]);
+    st.mx[j] = __builtin_elementwise_maximum(st.mx[j], v[j]);  // NaN stays
+  }
+}
+
+// Folds N tokens one after another, as decode steps do: the same sums whether a
 // block comes at once or a token at a time (the codes of fp8 entries hang on their
-// last bits).  Where v - max is NaN the weight is 1, as in pool_weight.
+// last bits).
 template <int N>
 __device__ __forceinline__ void pool_fold_serial(PoolLane& st, const float (&v)[N][8], const float (&c)[N][8]) {
 #pragma unroll
-  for (int u = 0; u < N; ++u) {
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float d = v[u][j] - st.mx[j];
-      const bool up = v[u][j] > st.mx[j];
-      const float t = d != d ? 1.f : expf(-__builtin_fabsf(d));  // rescales the state, or weighs the token
-      st.sum[j] = fmaf(t, up ? st.sum[j] : 1.f, up ? 1.f : st.sum[j]);
-      st.acc[j] = fmaf(t, up ? st.acc[j] : c[u][j], up ? c[u][j] : st.acc[j]);
-      st.mx[j] = __builtin_elementwise_maximum(st.mx[j], v[u][j]);  // NaN stays
-    }
-  }
+  for (int u = 0; u < N; ++u) pool_fold_token(st, v[u], c[u]);
 }
 
 // The state of a lane's channels seen from the larger max M[j]: sums and
