@@ -261,36 +261,25 @@ __device__ __forceinline__ void decode_fold_part(int m, int b, int64_t p, const 
       fold_bias(in, bias, pm, channels, grp);
     }
     const u32x4 b0 = in.b0, b1 = in.b1;
-    float mx[8], sum[8], acc[8], c[8], z[8], bb[8];
+    PoolLane st;
+    float c[8], v[8];
+    unpack8_bf16(in.cv, c);
+    unpack8_bf16(in.zv, v);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-      mx[j] = fresh ? -INFINITY : __uint_as_float(in.m0[j]);
-      mx[j + 4] = fresh ? -INFINITY : __uint_as_float(in.m1[j]);
-      sum[j] = fresh ? 0.f : __uint_as_float(in.s0[j]);
-      sum[j + 4] = fresh ? 0.f : __uint_as_float(in.s1[j]);
-      acc[j] = fresh ? 0.f : __uint_as_float(in.a0[j]);
-      acc[j + 4] = fresh ? 0.f : __uint_as_float(in.a1[j]);
-      bb[j] = __uint_as_float(b0[j]);
-      bb[j + 4] = __uint_as_float(b1[j]);
+      st.mx[j] = fresh ? -INFINITY : __uint_as_float(in.m0[j]);
+      st.mx[j + 4] = fresh ? -INFINITY : __uint_as_float(in.m1[j]);
+      st.sum[j] = fresh ? 0.f : __uint_as_float(in.s0[j]);
+      st.sum[j + 4] = fresh ? 0.f : __uint_as_float(in.s1[j]);
+      st.acc[j] = fresh ? 0.f : __uint_as_float(in.a0[j]);
+      st.acc[j + 4] = fresh ? 0.f : __uint_as_float(in.a1[j]);
+      v[j] += __uint_as_float(b0[j]);
+      v[j + 4] += __uint_as_float(b1[j]);
     }
-    unpack8_bf16(in.cv, c);
-    unpack8_bf16(in.zv, z);
+    pool_fold_token(st, v, c);
     float out[8];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      const float v = z[j] + bb[j];
-      if (v > mx[j]) {
-        const float sc = expf(mx[j] - v);
-        sum[j] = sum[j] * sc + 1.f;
-        acc[j] = acc[j] * sc + c[j];
-        mx[j] = v;
-      } else {
-        const float w = expf(v - mx[j]);
-        sum[j] += w;
-        acc[j] += w * c[j];
-      }
-      out[j] = mine ? acc[j] / sum[j] : 0.f;
-    }
+    for (int j = 0; j < 8; ++j) out[j] = mine ? pool_out(st, j) : 0.f;
 #pragma unroll
     for (int j = 0; j < 8; j += 2) bf16_round2(out[j], out[j + 1]);  // the compressor emits bf16 entries
     if (emit) {
@@ -300,14 +289,18 @@ __device__ __forceinline__ void decode_fold_part(int m, int b, int64_t p, const 
       }
     } else if (mine) {
       u32x4* wp = reinterpret_cast<u32x4*>(sbase + grp * 8);
-      wp[0] = u32x4{__float_as_uint(mx[0]), __float_as_uint(mx[1]), __float_as_uint(mx[2]), __float_as_uint(mx[3])};
-      wp[1] = u32x4{__float_as_uint(mx[4]), __float_as_uint(mx[5]), __float_as_uint(mx[6]), __float_as_uint(mx[7])};
       u32x4* ws = reinterpret_cast<u32x4*>(sbase + channels + grp * 8);
-      ws[0] = u32x4{__float_as_uint(sum[0]), __float_as_uint(sum[1]), __float_as_uint(sum[2]), __float_as_uint(sum[3])};
-      ws[1] = u32x4{__float_as_uint(sum[4]), __float_as_uint(sum[5]), __float_as_uint(sum[6]), __float_as_uint(sum[7])};
       u32x4* wa = reinterpret_cast<u32x4*>(sbase + 2 * channels + grp * 8);
-      wa[0] = u32x4{__float_as_uint(acc[0]), __float_as_uint(acc[1]), __float_as_uint(acc[2]), __float_as_uint(acc[3])};
-      wa[1] = u32x4{__float_as_uint(acc[4]), __float_as_uint(acc[5]), __float_as_uint(acc[6]), __float_as_uint(acc[7])};
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const auto half = [i](const float (&x)[8]) {
+          return u32x4{__float_as_uint(x[4 * i]), __float_as_uint(x[4 * i + 1]), __float_as_uint(x[4 * i + 2]),
+                       __float_as_uint(x[4 * i + 3])};
+        };
+        wp[i] = half(st.mx);
+        ws[i] = half(st.sum);
+        wa[i] = half(st.acc);
+      }
     }
   }
 }

@@ -63,8 +63,9 @@ __device__ __forceinline__ void pool_fold(PoolLane& st, const float (&v)[N][8], 
   }
 }
 
-// Folds one token (values v, rows c).  Where v - max is NaN the weight is 1, as in
-// pool_weight.
+// Folds one token (values v, rows c).  Appends and decode steps fold with it in
+// turn, so that a state which one of them leaves means the same to the other.
+// Where v - max is NaN the weight is 1, as in pool_weight.
 __device__ __forceinline__ void pool_fold_token(PoolLane& st, const float (&v)[8], const float (&c)[8]) {
 #pragma unroll
   for (int j = 0; j < 8; ++j) {
