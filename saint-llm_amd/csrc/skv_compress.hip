@@ -11,9 +11,10 @@
 //   FP8 quantize-on-write (quant/reference.py:75-110) on each 128-dim block.
 // Here the buffered state of the incomplete block is the running online-softmax
 // state of each channel (max, sum, weighted sum; fp32 [batch, 3, channels]),
-// so a decode step costs O(channels) whatever m is, and a block emits from
-// that state the same value a one-shot pooling of its m tokens gives.
+// so a decode step costs O(channels) whatever m is, and a block emits the same
+// bits whichever calls brought its m tokens.
 #include <algorithm>
+#include <type_traits>
 
 #include "skv_pool_state.h"
 
@@ -42,165 +43,168 @@ struct CompressArgs {
   int fp8_main;  // main (quantized) channels in FP8 format
 };
 
-// Work split.  The pooling is independent per channel, so a workgroup takes a
-// block of 128 channels (one fp8 scale block): 16 lanes of 8 channels read
-// 256 consecutive bytes of a token row, and the 16 lane groups of its 4 waves
-// are shared out between entries and token slices.  kSlices lane groups fold
-// the tokens of one entry in turn, 4 tokens of a lane in flight at once, and
-// are merged by lane shuffles (and through LDS for 16 slices); the other lane
-// groups hold other entries.  A block of 4 tokens needs no slices (16 entries
-// per workgroup); one of 128 takes all 16 lane groups, 8 tokens each.
-// HBM-bound: c and z rows are read once.  One wave folding an entry's tokens one
-// after another, with a memory round trip each, took 1.45 us per token.  4
-// sequences of 6,700-8,192 tokens x 576 bf16 channels: entries of 4 tokens 33 us
-// (2.6 TB/s; the call averaged 247 us before; 25 with the weights of a turn taken
-// against its max at once, which moves the last bits of the sums and so codes of
-// fp8 entries), of 128 tokens 26 us; 16 x 8,192 tokens in entries of 4 110 us; two
-// sequences of 95 and 300 tokens 5.5 and, with blocks of 128, 8.3 us (186 before).
+// Work split.  The pooling is independent per channel and serial over an entry's
+// tokens, so a row of lanes takes 128 channels (one fp8 scale block) of one entry,
+// kCh of them a lane, and the rows of a workgroup's 4 waves are shared out between
+// entries and blocks of channels.
+//   * kCh = 8 (16 lanes read 256 consecutive bytes of a token row) where a call
+//     brings an entry at most 4 tokens, which are in flight at once.
+//   * Of longer entries the chain of tokens sets the time, about 26 instructions a
+//     token and channel: 0.1 us a token at one channel a lane (2 waves a row), which
+//     is taken while the rows are too few to fill the SIMDs.  With 8 rows per CU and
+//     more the loads count: 8 channels up to 15 tokens, then 2.
+// HBM-bound where the device is full: c and z rows are read once.  bf16 rows of 576
+// channels, against one wave per entry with a memory round trip a token: 4
+// sequences of 8,192 tokens in entries of 4 tokens 31 us (2.7 TB/s; 145), of 32 28
+// (121), of 128 33 (455; at 2 channels a lane 38); two of 300 tokens in entries of 4
+// 7.5 (17.6), of 128 19 (515).  (An entry's tokens split over 16 rows of lanes took
+// 9.4 us there and 24 above, but its sums hung on how the tokens came.)
 constexpr int kCmThreads = 256;
-constexpr int kCmWaves = kCmThreads / kWave;
-constexpr int kCmLanes = 16;                         // lanes per 128-channel token row
-constexpr int kCmGroups = kCmThreads / kCmLanes;     // lane groups per workgroup
-constexpr int kCmFold = 4;                           // tokens in flight per lane
+constexpr int kCmBlock = 128;  // channels of a row of lanes
+constexpr int kCmRows = 4;     // most rows of 1 or 2 channels a lane
 
-struct CompressSmem {
-  float mx[kCmWaves][8][kCmLanes];  // of 16 slices: each wave's max, then its sums from the common max
-  float sum[kCmWaves - 1][8][kCmLanes], acc[kCmWaves - 1][8][kCmLanes];
-};
-
-// A lane's 8 channels of a row as they lie in memory (bf16 or fp32).
-template <class Row>
+// A lane's kCh channels of a row as they lie in memory (bf16 or fp32).
+template <class Row, int kCh>
 struct RawRow {
-  static constexpr int kVecs = sizeof(Row) / 2;  // 16-byte pieces
-  u32x4 v[kVecs];
+  static constexpr int kWords = (kCh * sizeof(Row) + 3) / 4;
+  uint32_t w[kWords];
   __device__ __forceinline__ void load(const uint8_t* row, int grp) {
-    const u32x4* p = reinterpret_cast<const u32x4*>(row + grp * 16 * kVecs);
+    const uint8_t* p = row + grp * static_cast<int>(kCh * sizeof(Row));
+    if constexpr (kCh == 8) {
 #pragma unroll
-    for (int i = 0; i < kVecs; ++i) v[i] = p[i];
-  }
-  __device__ __forceinline__ void get(float* f) const {
-    if constexpr (kVecs == 1) {
-      unpack8_bf16(v[0], f);
+      for (int i = 0; i < kWords; i += 4) {
+        const u32x4 x = *reinterpret_cast<const u32x4*>(p + 4 * i);
+#pragma unroll
+        for (int j = 0; j < 4; ++j) w[i + j] = x[j];
+      }
     } else {
+      using Piece = std::conditional_t<kCh * sizeof(Row) == 8, u32x2, std::conditional_t<kCh * sizeof(Row) == 4, uint32_t, uint16_t>>;
+      const Piece x = *reinterpret_cast<const Piece*>(p);
+      if constexpr (kWords == 2) {
+        w[0] = x[0];
+        w[1] = x[1];
+      } else {
+        w[0] = x;
+      }
+    }
+  }
+  __device__ __forceinline__ void get(float (&f)[kCh]) const {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) f[j] = __uint_as_float(v[j >> 2][j & 3]);
+    for (int j = 0; j < kCh; ++j) {
+      if constexpr (sizeof(Row) == 2) {
+        f[j] = __uint_as_float(j & 1 ? w[j / 2] & 0xffff0000u : w[j / 2] << 16);
+      } else {
+        f[j] = __uint_as_float(w[j]);
+      }
     }
   }
 };
 
-// Tokens first + slice + stride * i < p1 of entry e (sequence b) folded into
-// st.  Every load of a turn is issued before any is used (left to itself the
+// kFold tokens of an entry, their loads issued together (left to itself the
 // compiler waits for each row in turn: 14.8 us for a call of a few entries).
-template <class Row, bool kSerial>
-__device__ __forceinline__ void fold_tokens(PoolLane& st, const CompressArgs& a, int b, int first_new, int e, int first,
-                                            int p1, int slice, int stride, int grp) {
-  typedef float f32x4u __attribute__((ext_vector_type(4), aligned(4)));  // bias is 4-byte aligned
-  const uint8_t* cbase = a.c_new + b * a.in_seq_stride;
-  const uint8_t* zbase = a.z_new + b * a.in_seq_stride;
-  for (int p = first + slice; p < p1; p += kCmFold * stride) {
-    RawRow<Row> cr[kCmFold], zr[kCmFold];
-    f32x4u br[kCmFold][2];
-    bool live[kCmFold];
+template <class Row, int kCh>
+struct FoldTurn {
+  static constexpr int kFold = kCh == 8 ? 4 : 16 / kCh;
+  static constexpr int kVec = kCh == 8 ? 4 : kCh;
+  typedef float f32v __attribute__((ext_vector_type(kVec), aligned(4)));  // bias is 4-byte aligned
+  RawRow<Row, kCh> c[kFold], z[kFold];
+  f32v bias[kFold][kCh / kVec];
+
+  // tokens p, p + 1, ... below p1 of entry e (sequence b), channels kCh grp on
+  __device__ __forceinline__ void load(const CompressArgs& a, int b, int first_new, int e, int p, int p1, int grp) {
+    const int64_t at = b * a.in_seq_stride + (p - first_new) * a.in_row_stride;
+    const uint8_t *cp = a.c_new + at, *zp = a.z_new + at;
+    const float* bp = a.bias + static_cast<int64_t>(p - e * a.m) * a.channels + grp * kCh;
 #pragma unroll
-    for (int u = 0; u < kCmFold; ++u) {
-      const int pu = p + u * stride;
-      live[u] = pu < p1;
-      const int q = live[u] ? pu : p;  // a row that exists
-      const int64_t off = (q - first_new) * a.in_row_stride;
-      zr[u].load(zbase + off, grp);
-      cr[u].load(cbase + off, grp);
-      const f32x4u* bp = reinterpret_cast<const f32x4u*>(a.bias + static_cast<int64_t>(q - e * a.m) * a.channels + grp * 8);
-      br[u][0] = bp[0];
-      br[u][1] = bp[1];
+    for (int u = 0; u < kFold; ++u) {  // past the last token: its row again
+      z[u].load(zp, grp);
+      c[u].load(cp, grp);
+#pragma unroll
+      for (int i = 0; i < kCh / kVec; ++i) bias[u][i] = reinterpret_cast<const f32v*>(bp)[i];
+      const bool on = p + u + 1 < p1;
+      zp += on ? a.in_row_stride : 0;
+      cp += on ? a.in_row_stride : 0;
+      bp += on ? a.channels : 0;
     }
     __builtin_amdgcn_sched_barrier(0);
-    float v[kCmFold][8], c[kCmFold][8];
+  }
+  __device__ __forceinline__ void values(int u, float (&v)[kCh]) const {
+    z[u].get(v);
 #pragma unroll
-    for (int u = 0; u < kCmFold; ++u) {
-      zr[u].get(v[u]);
-      cr[u].get(c[u]);
+    for (int j = 0; j < kCh; ++j) v[j] += bias[u][j / kVec][j % kVec];
+  }
+};
+
+// Tokens [p, p1), at least one, of entry e (sequence b) folded into st, 8 channels a lane.
+template <class Row>
+__device__ __forceinline__ void fold_tokens(PoolLane<8>& st, const CompressArgs& a, int b, int first_new, int e, int p,
+                                            int p1, int grp) {
+  using Turn = FoldTurn<Row, 8>;
+  for (; p < p1; p += Turn::kFold) {
+    Turn t;
+    t.load(a, b, first_new, e, p, p1, grp);
+    const auto one = [&](int u) {
+      float v[8], x[8];
+      t.values(u, v);
+      t.c[u].get(x);
+      pool_fold_token(st, v, x);
+    };
+    if (__ballot(p1 - p < Turn::kFold)) {  // a turn past some lane's last token
 #pragma unroll
-      for (int j = 0; j < 8; ++j) v[u][j] += br[u][j >> 2][j & 3];
-    }
-    const bool part = __ballot(!live[kCmFold - 1]);  // a turn past some lane's last token
-    if constexpr (kSerial) {
-      if (part) {
-#pragma unroll
-        for (int u = 0; u < kCmFold; ++u) {
-          if (live[u]) pool_fold_token(st, v[u], c[u]);
-        }
-      } else {
-        pool_fold_serial<kCmFold>(st, v, c);
+      for (int u = 0; u < Turn::kFold; ++u) {
+        if (u < p1 - p) one(u);
       }
     } else {
-      if (part) {  // tokens past the end: value -inf whatever the bias, row -0: nothing is added
 #pragma unroll
-        for (int u = 1; u < kCmFold; ++u) {
-#pragma unroll
-          for (int j = 0; j < 8; ++j) {
-            v[u][j] = live[u] ? v[u][j] : -INFINITY;
-            c[u][j] = live[u] ? c[u][j] : -0.f;
-          }
-        }
-      }
-      pool_fold<kCmFold>(st, v, c);
+      for (int u = 0; u < Turn::kFold; ++u) one(u);
     }
   }
 }
 
-// The states of the lane groups of one entry, merged: every lane group holds
-// the result for 1 and 4 slices (one lane group, one wave), wave 0 for 16.
-// For 16 slices every thread of the workgroup must call it.
-template <int kSlices>
-__device__ __forceinline__ void merge_slices(CompressSmem& sm, PoolLane& st) {
-  static_assert(kSlices == 1 || kSlices == 4 || kSlices == 16, "one lane group, one wave or the workgroup");
-  if constexpr (kSlices == 1) return;
-  float M[8];
+// The same, kCh = 1 or 2 channels a lane of a whole wave (p uniform).  A turn's
+// weights come first, off the chain: the maximum that a token meets does not wait
+// for the sums.  The next turn's loads are in flight meanwhile.
+template <class Row, int kCh>
+__device__ __forceinline__ void fold_tokens(PoolLane<kCh>& st, const CompressArgs& a, int b, int first_new, int e, int p,
+                                            int p1, int grp) {
+  using Turn = FoldTurn<Row, kCh>;
+  Turn t;
+  t.load(a, b, first_new, e, p, p1, grp);
+  for (;;) {
+    float v[Turn::kFold][kCh], x[Turn::kFold][kCh];
 #pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    M[j] = __builtin_elementwise_maximum(st.mx[j], __shfl_xor(st.mx[j], 16));
-    M[j] = __builtin_elementwise_maximum(M[j], __shfl_xor(M[j], 32));
-  }
-  pool_rebase(st, M);
-#pragma unroll
-  for (int j = 0; j < 8; ++j) {
-    st.sum[j] += __shfl_xor(st.sum[j], 16);
-    st.acc[j] += __shfl_xor(st.acc[j], 16);
-    st.sum[j] += __shfl_xor(st.sum[j], 32);
-    st.acc[j] += __shfl_xor(st.acc[j], 32);
-  }
-  if constexpr (kSlices == 16) {
-    const int wave = threadIdx.x / kWave, l = threadIdx.x % kCmLanes;
-    if (threadIdx.x % kWave < kCmLanes) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) sm.mx[wave][j][l] = st.mx[j];
+    for (int u = 0; u < Turn::kFold; ++u) {
+      t.values(u, v[u]);
+      t.c[u].get(x[u]);
     }
-    __syncthreads();
+    const int n = p1 - p;
+    p += Turn::kFold;
+    if (p < p1) t.load(a, b, first_new, e, p, p1, grp);
+    const auto fold = [&](auto live) {
+      float w[Turn::kFold][kCh];
+      bool up[Turn::kFold][kCh];
 #pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      M[j] = sm.mx[0][j][l];
+      for (int u = 0; u < Turn::kFold; ++u) {
 #pragma unroll
-      for (int w = 1; w < kCmWaves; ++w) M[j] = __builtin_elementwise_maximum(M[j], sm.mx[w][j][l]);
-    }
-    pool_rebase(st, M);
-    if (wave > 0 && threadIdx.x % kWave < kCmLanes) {
-#pragma unroll
-      for (int j = 0; j < 8; ++j) {
-        sm.sum[wave - 1][j][l] = st.sum[j];
-        sm.acc[wave - 1][j][l] = st.acc[j];
-      }
-    }
-    __syncthreads();
-    if (wave == 0) {
-#pragma unroll
-      for (int w = 0; w < kCmWaves - 1; ++w) {
-#pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          st.sum[j] += sm.sum[w][j][l];
-          st.acc[j] += sm.acc[w][j][l];
+        for (int j = 0; j < kCh; ++j) {
+          const float vu = live(u) ? v[u][j] : -INFINITY;  // past the end: leaves the maximum as it is
+          w[u][j] = pool_weight(vu, st.mx[j], up[u][j]);
+          st.mx[j] = __builtin_elementwise_maximum(st.mx[j], vu);  // NaN stays
         }
       }
+#pragma unroll
+      for (int u = 0; u < Turn::kFold; ++u) {
+        if (!live(u)) continue;
+#pragma unroll
+        for (int j = 0; j < kCh; ++j) pool_add(st.sum[j], st.acc[j], w[u][j], up[u][j], x[u][j]);
+      }
+    };
+    if (n >= Turn::kFold) {
+      fold([](int) { return true; });
+    } else {
+      fold([n](int u) { return u < n; });
     }
+    if (p >= p1) return;
   }
 }
 
@@ -211,11 +215,11 @@ __device__ __forceinline__ int32_t entry_page(const CompressArgs& a, int b, int 
 }
 
 // Entry e, in page `page` of its table, from its channels' states (16 lanes, 8 channels each).
-__device__ __forceinline__ void emit_entry(const PoolLane& st, const CompressArgs& a, int e, int32_t page, int grp,
-                                           int groups) {
+__device__ __forceinline__ void emit_entry(const PoolLane<8>& st, const CompressArgs& a, int e, int32_t page, int grp) {
   const int page_idx = e / a.bs;
-  if (page_idx >= a.bt_stride || page < 0 || page >= a.n_pages) return;  // uniform over the lane group
+  if (page_idx >= a.bt_stride || page < 0 || page >= a.n_pages) return;  // uniform over the row of lanes
   uint8_t* entry = a.pool + (static_cast<int64_t>(page) * a.bs + (e - page_idx * a.bs)) * a.entry_bytes;
+  const int groups = a.channels >> 3;
   float out[8];
 #pragma unroll
   for (int j = 0; j < 8; ++j) out[j] = grp < groups ? pool_out(st, j) : 0.f;
@@ -226,70 +230,114 @@ __device__ __forceinline__ void emit_entry(const PoolLane& st, const CompressArg
   store_entry_group(entry, out, grp, groups, a.format, a.fp8_main);
 }
 
-// One workgroup of a stream: workgroup bx of gx over the blocks of sequence b,
-// 128-channel block zb.  Blocks
-// [e0, e1) of a sequence complete in this call; block e0 continues from the
-// stored state when the call before left it incomplete, and the tokens of
-// block e1, when it stays incomplete, go to the state.  When one call does
-// both for different blocks, workgroup 0 takes block e1 in a turn of its own
-// after block e0 (which is its first), so that the state is read before it
-// is written.
-template <class Row, int kSlices>
-__device__ __forceinline__ void compress_workgroup(CompressSmem& sm, const CompressArgs& a, int bx, int gx, int b, int zb) {
-  constexpr int kEntries = kCmGroups / kSlices;  // per workgroup and turn
-  const int L = a.lens[b];
-  const int n = a.n_new ? a.n_new[b] : a.n_uni;
-  if (n <= 0 || n > L || n > a.in_len) return;
-  const int first_new = L - n;
-  const int e0 = first_new / a.m;
-  const int e1 = L / a.m;
-  const bool resumes = first_new > e0 * a.m;  // block e0 has a stored state
-  const bool leaves = L > e1 * a.m;           // block e1 leaves one
-  bool last_turn = bx == 0 && resumes && leaves && e1 > e0;
-  const int n_units = e1 - e0 + (leaves && !(resumes && e1 > e0) ? 1 : 0);
-  const int groups = a.channels >> 3;
-  const int grp = zb * kCmLanes + threadIdx.x % kCmLanes;
+// The blocks that a sequence's new tokens touch: blocks [e0, e1) complete in this
+// call; block e0 continues from the stored state when the call before left it
+// incomplete, and the tokens of block e1, when it stays incomplete, go to the
+// state.  When one call does both for different blocks, workgroup 0 takes block e1
+// in a turn of its own after block e0 (which is its first), so that the state is
+// read before it is written.
+struct CompressSpan {
+  int L, first_new, e0, e1;
+  bool resumes, leaves;  // block e0 has a stored state; block e1 leaves one
+  int n_units;           // blocks without that last turn's
+  __device__ __forceinline__ bool load(const CompressArgs& a, int b) {
+    L = __builtin_amdgcn_readfirstlane(a.lens[b]);
+    const int n = a.n_new ? __builtin_amdgcn_readfirstlane(a.n_new[b]) : a.n_uni;
+    if (n <= 0 || n > L || n > a.in_len) return false;
+    first_new = L - n;
+    e0 = first_new / a.m;
+    e1 = L / a.m;
+    resumes = first_new > e0 * a.m;
+    leaves = L > e1 * a.m;
+    n_units = e1 - e0 + (leaves && !apart() ? 1 : 0);
+    return true;
+  }
+  __device__ __forceinline__ bool apart() const { return resumes && leaves && e1 > e0; }
+  __device__ __forceinline__ int from(const CompressArgs& a, int e) const { return max(first_new, e * a.m); }
+  __device__ __forceinline__ int to(const CompressArgs& a, int e) const {
+    return static_cast<int>(min<int64_t>(L, (e + 1) * static_cast<int64_t>(a.m)));
+  }
+};
+
+struct CompressSmem {
+  alignas(16) float state[kCmRows][3][kCmBlock];  // a completed entry's (max, sum, weighted sum)
+};
+
+// Workgroup bx of gx over the blocks of sequence b of a stream, the zz-th part of
+// its channels; its rows of lanes are `slots` entries of as many 128-channel blocks
+// as remain.
+template <class Row, int kCh>
+__device__ __forceinline__ void compress_workgroup(CompressSmem& sm, const CompressArgs& a, int bx, int gx, int b, int zz,
+                                                   int slots) {
+  constexpr int kLanes = kCmBlock / kCh, kRows = kCmThreads / kLanes;
+  CompressSpan sp;
+  if (!sp.load(a, b)) return;
+  const bool last_turn = bx == 0 && sp.apart();
+  // rows of whole waves: known uniform, so that their addresses are scalars
+  const int row = (kCh == 8 ? static_cast<int>(threadIdx.x) : __builtin_amdgcn_readfirstlane(threadIdx.x)) / kLanes;
+  const int zper = kRows / slots, slot = row / zper;
+  const int grp0 = (zz * zper + row % zper) * kLanes, grp = grp0 + threadIdx.x % kLanes;
+  const int groups = a.channels / kCh;
   const int gsafe = min(grp, groups - 1);  // lanes past the channels read the last group and store nothing
-  const int slot = threadIdx.x / kCmLanes / kSlices, slice = threadIdx.x / kCmLanes % kSlices;
-  float* sbase = a.state + static_cast<int64_t>(b) * 3 * a.channels + gsafe * 8;
-  int unit0 = bx * kEntries;
-  while (unit0 < n_units || last_turn) {
-    const bool in_last = unit0 >= n_units;
+  float* sbase = a.state + static_cast<int64_t>(b) * 3 * a.channels + gsafe * kCh;
+  int unit0 = bx * slots;
+  while (unit0 < sp.n_units || last_turn) {
+    const bool in_last = unit0 >= sp.n_units;
     if (in_last) __syncthreads();  // block e0's lanes have read the state
-    const int unit = in_last ? e1 - e0 + slot : unit0 + slot;
-    const int e = e0 + unit;
-    const bool active = in_last ? slot == 0 : unit < n_units;
-    PoolLane st;
-    pool_reset(st);
+    const int e = in_last ? sp.e1 + slot : sp.e0 + unit0 + slot;
+    const bool active = grp0 < groups && (in_last ? slot == 0 : unit0 + slot < sp.n_units);  // uniform over the row of lanes
     int32_t page = -1;
     if (active) {
       page = entry_page(a, b, e);
-      if (e == e0 && slice == 0 && resumes) {
+      PoolLane<kCh> st;
+      pool_reset(st);
+      if (e == sp.e0 && sp.resumes) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+        for (int j = 0; j < kCh; ++j) {
           st.mx[j] = sbase[j];
           st.sum[j] = sbase[a.channels + j];
           st.acc[j] = sbase[2 * a.channels + j];
         }
       }
-      fold_tokens<Row, kSlices == 1>(st, a, b, first_new, e, max(first_new, e * a.m), min(L, (e + 1) * a.m), slice, kSlices, gsafe);
-    }
-    merge_slices<kSlices>(sm, st);
-    if (active && slice == 0) {
-      if (e < e1) {
-        emit_entry(st, a, e, page, grp, groups);
+      fold_tokens<Row>(st, a, b, sp.first_new, e, sp.from(a, e), sp.to(a, e), gsafe);
+      if (e < sp.e1) {
+        if constexpr (kCh == 8) {
+          emit_entry(st, a, e, page, grp);
+        } else {
+          const int i = threadIdx.x % kLanes;
+#pragma unroll
+          for (int j = 0; j < kCh; ++j) {
+            sm.state[row][0][kCh * i + j] = st.mx[j];
+            sm.state[row][1][kCh * i + j] = st.sum[j];
+            sm.state[row][2][kCh * i + j] = st.acc[j];
+          }
+        }
       } else if (grp < groups) {
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
+        for (int j = 0; j < kCh; ++j) {
           sbase[j] = st.mx[j];
           sbase[a.channels + j] = st.sum[j];
           sbase[2 * a.channels + j] = st.acc[j];
         }
       }
     }
+    if constexpr (kCh < 8) {  // the entry by 16 lanes of 8 channels
+      __syncthreads();
+      const int i = threadIdx.x % kLanes;
+      if (active && e < sp.e1 && i < kCmBlock / 8) {
+        PoolLane<8> st;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+          st.mx[j] = sm.state[row][0][8 * i + j];
+          st.sum[j] = sm.state[row][1][8 * i + j];
+          st.acc[j] = sm.state[row][2][8 * i + j];
+        }
+        emit_entry(st, a, e, page, grp0 * kCh / 8 + i);
+      }
+      if (unit0 + gx * slots < sp.n_units) __syncthreads();  // the LDS is written again
+    }
     if (in_last) break;
-    unit0 += gx * kEntries;
-    if constexpr (kSlices == 16) __syncthreads();  // the LDS is written again
+    unit0 += gx * slots;
   }
 }
 
@@ -304,8 +352,9 @@ struct CompressStreams {
   CompressArgs s[kCmStreams];
   int32_t first[kCmStreams];  // first workgroup
   int32_t turns[kCmStreams];  // workgroups over a sequence's blocks
-  int32_t zblocks[kCmStreams];
-  int32_t slices[kCmStreams];
+  int32_t zparts[kCmStreams];  // workgroups over the channels
+  int32_t slots[kCmStreams];   // entries of a workgroup at a time
+  int32_t channels[kCmStreams];  // of a lane: 8, 2 or 1
   int32_t n, batch;
 };
 
@@ -316,12 +365,14 @@ __global__ __launch_bounds__(kCmThreads, sizeof(Row) == 2 ? 3 : 2) void k_compre
   while (i + 1 < cs.n && static_cast<int>(blockIdx.x) >= cs.first[i + 1]) ++i;  // uniform
   const CompressArgs& a = cs.s[i];
   const int l = blockIdx.x - cs.first[i];
-  const int rest = l / cs.zblocks[i], zb = l - rest * cs.zblocks[i];
+  const int rest = l / cs.zparts[i], zz = l - rest * cs.zparts[i];
   const int b = rest / cs.turns[i], bx = rest - b * cs.turns[i];
-  switch (cs.slices[i]) {  // uniform
-    case 1: compress_workgroup<Row, 1>(sm, a, bx, cs.turns[i], b, zb); break;
-    case 4: compress_workgroup<Row, 4>(sm, a, bx, cs.turns[i], b, zb); break;
-    default: compress_workgroup<Row, 16>(sm, a, bx, cs.turns[i], b, zb); break;
+  if (cs.channels[i] == 8) {  // uniform
+    compress_workgroup<Row, 8>(sm, a, bx, cs.turns[i], b, zz, cs.slots[i]);
+  } else if (cs.channels[i] == 2) {
+    compress_workgroup<Row, 2>(sm, a, bx, cs.turns[i], b, zz, cs.slots[i]);
+  } else {
+    compress_workgroup<Row, 1>(sm, a, bx, cs.turns[i], b, zz, cs.slots[i]);
   }
 }
 
@@ -414,21 +465,24 @@ static int compress_streams(const char* what, const skv_compress_stream* streams
     }
     if (cs.n == 0) blocks = 0;
     run_f32 = f32;
-    // slices of an entry: at least 4 tokens per lane, which a turn of fold_tokens takes at once
-    // (blocks of 8 over 4 slices: 54 us for 4 x 8192 tokens of 576 channels, over one: 24 us)
-    const int slices = a.m < 16 ? 1 : a.m < 64 ? 4 : 16;
-    const int64_t zblocks = ceil_div(a.channels, 8 * kCmLanes);
-    // a call's tokens lie in at most ceil(in_len / m) + 1 blocks; past 2^26
+    // a call's tokens lie in at most ceil((in_len - 1) / m) + 1 blocks; past 2^26
     // workgroups of a stream each takes several turns
-    const int64_t turns = std::min<int64_t>(ceil_div(ceil_div(a.in_len, a.m) + 1, kCmGroups / slices),
-                                            std::max<int64_t>(1, (1 << 26) / (batch * zblocks)));
+    // a call's tokens lie in at most ceil((in_len - 1) / m) + 1 blocks; past 2^26
+    // workgroups of a stream each takes several turns
+    const int64_t units = ceil_div(a.in_len - 1, a.m) + 1, zblocks = ceil_div(a.channels, kCmBlock);
+    const int64_t tokens = std::min<int64_t>(a.m, a.in_len);  // most of an entry
+    const int ch = tokens <= 4 ? 8 : units * batch * zblocks < 8 * device_cus() ? 1 : tokens < 16 ? 8 : 2;
+    const int rows = kCmThreads * ch / kCmBlock, slots = rows;
+    const int64_t zparts = ceil_div(zblocks, rows / slots);
+    const int64_t turns = std::min<int64_t>(ceil_div(units, slots), std::max<int64_t>(1, (1 << 26) / (batch * zparts)));
     cs.s[cs.n] = a;
     cs.first[cs.n] = static_cast<int32_t>(blocks);
     cs.turns[cs.n] = static_cast<int32_t>(turns);
-    cs.zblocks[cs.n] = static_cast<int32_t>(zblocks);
-    cs.slices[cs.n] = slices;
+    cs.zparts[cs.n] = static_cast<int32_t>(zparts);
+    cs.slots[cs.n] = slots;
+    cs.channels[cs.n] = ch;
     ++cs.n;
-    blocks += turns * batch * zblocks;
+    blocks += turns * batch * zparts;
   }
   return launch_streams(what, cs, blocks, run_f32, stream);
 }

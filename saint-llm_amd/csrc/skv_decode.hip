@@ -261,7 +261,7 @@ __device__ __forceinline__ void decode_fold_part(int m, int b, int64_t p, const 
       fold_bias(in, bias, pm, channels, grp);
     }
     const u32x4 b0 = in.b0, b1 = in.b1;
-    PoolLane st;
+    PoolLane<8> st;
     float c[8], v[8];
     unpack8_bf16(in.cv, c);
     unpack8_bf16(in.zv, v);
