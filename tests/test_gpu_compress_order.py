@@ -72,3 +72,31 @@ def test_decode_steps_give_the_prompt_bits(dev, m, fp8) -> None:
             assert torch.equal(x, y), (q, e)
         if n % m:
             assert torch.equal(caches[0].state[0][q], caches[1].state[0][q]), q
+
+
+@pytest.mark.parametrize("m,t,ch,rows", [(4, 1, 576, torch.bfloat16), (4, 3, 2048, torch.bfloat16),
+                                         (128, 1, 136, torch.float32), (32, 6, 576, torch.float32),
+                                         (16, 40, 264, torch.bfloat16)])
+def test_many_sequences_at_once(dev, m, t, ch, rows) -> None:
+    """Workgroups shared by several blocks of channels give the bits of calls of a few sequences."""
+    from saint_kv import ops
+
+    g = torch.Generator().manual_seed(m + t)
+    b, part, had = 513, 3, 2  # the blocks hold two tokens before the call
+    c, z = (torch.randn(b, had + t, ch, generator=g).to(dev, rows) for _ in range(2))
+    bias = torch.randn(m, ch, generator=g).to(dev)
+    new = torch.randint(0, t + 1, (b,), generator=g, dtype=torch.int32).to(dev)
+    got = []
+    for size in (b, part):
+        pool = torch.zeros(b, 16, ch, dtype=torch.bfloat16, device=dev)
+        state = torch.zeros(b, 3, ch, device=dev)
+        for lo in range(0, b, size):
+            at = slice(lo, min(lo + size, b))
+            bt = _i32([[i] for i in range(lo, at.stop)], dev)
+            n = new[at]
+            ops.compress_append(pool, bt, state[at], c[at, :had], z[at, :had], bias, torch.full_like(n, had), had)
+            ops.compress_append(pool, bt, state[at], c[at, had:], z[at, had:], bias, n + had, n)
+        got.append((pool, state))
+    assert torch.equal(got[0][0], got[1][0])
+    live = (had + new) % m > 0  # a state is left
+    assert torch.equal(got[0][1][live], got[1][1][live]) and bool(live.any())
