@@ -347,6 +347,12 @@ __device__ __forceinline__ void compress_workgroup(CompressSmem& sm, const Compr
 // streams (three layers; 4 prompts of 6,700-8,192 tokens): 112 us in five launches,
 // 73 in one (3.1 TB/s).
 constexpr int kCmStreams = 16;
+// Workgroups of a stream (65,535 sequences of 16 blocks of channels are fewer).  All
+// streams together keep below the 2^32 threads of a launch, past which the runtime
+// starts the remainder only and reports no error.
+constexpr int64_t kCmMaxBlocks = (1 << 20) - 1;
+static_assert(65535 * (kPoolWave * 8 * kMaxGroups / kCmBlock) <= kCmMaxBlocks &&
+              kCmStreams * kCmMaxBlocks * kCmThreads < int64_t(1) << 32, "one launch");
 
 struct CompressStreams {
   CompressArgs s[kCmStreams];
@@ -465,10 +471,8 @@ static int compress_streams(const char* what, const skv_compress_stream* streams
     }
     if (cs.n == 0) blocks = 0;
     run_f32 = f32;
-    // a call's tokens lie in at most ceil((in_len - 1) / m) + 1 blocks; past 2^26
-    // workgroups of a stream each takes several turns
-    // a call's tokens lie in at most ceil((in_len - 1) / m) + 1 blocks; past 2^26
-    // workgroups of a stream each takes several turns
+    // a call's tokens lie in at most ceil((in_len - 1) / m) + 1 blocks
+    // a call's tokens lie in at most ceil((in_len - 1) / m) + 1 blocks
     const int64_t units = ceil_div(a.in_len - 1, a.m) + 1, zblocks = ceil_div(a.channels, kCmBlock);
     const int64_t tokens = std::min<int64_t>(a.m, a.in_len);  // most of an entry
     const int ch = tokens <= 4 ? 8 : units * batch * zblocks < 8 * device_cus() ? 1 : tokens < 16 ? 8 : 2;
@@ -481,7 +485,8 @@ static int compress_streams(const char* what, const skv_compress_stream* streams
     while (slots < rows && slots < units) slots *= 2;
     if (batch * ceil_div(units, slots) * ceil_div(zblocks, rows / slots) < device_cus()) slots = rows;
     const int64_t zparts = ceil_div(zblocks, rows / slots);
-    const int64_t turns = std::min<int64_t>(ceil_div(units, slots), std::max<int64_t>(1, (1 << 26) / (batch * zparts)));
+    // past its share of a launch's workgroups each of a stream's takes several turns
+    const int64_t turns = std::min<int64_t>(ceil_div(units, slots), std::max<int64_t>(1, kCmMaxBlocks / (batch * zparts)));
     cs.s[cs.n] = a;
     cs.first[cs.n] = static_cast<int32_t>(blocks);
     cs.turns[cs.n] = static_cast<int32_t>(turns);
