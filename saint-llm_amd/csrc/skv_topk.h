@@ -202,8 +202,8 @@ constexpr size_t topk_bucket_lds(int k) {
   return need > sizeof(TopkBucketSmem<kThreads>) ? need : sizeof(TopkBucketSmem<kThreads>);
 }
 
-// emit(j, v) as topk_row_emit calls it.  kRegs: at most kThreads * kTbPer valid scores.
-template <int kThreads, bool kRegs, class Emit>
+// emit(j, v) as topk_row_emit calls it.
+template <int kThreads, class Emit>
 __device__ __forceinline__ void topk_row_buckets(TopkBucketSmem<kThreads>& sm, const float* row, int n_cols, int n_valid,
                                                  int k, Emit emit) {
   const int tid = threadIdx.x;
@@ -213,11 +213,12 @@ __device__ __forceinline__ void topk_row_buckets(TopkBucketSmem<kThreads>& sm, c
   for (int j = sel + tid; j < k; j += kThreads) emit(j, -1);
   if (sel == 0) return;
   const float inf = __builtin_huge_valf();
+  const bool fits = n_valid <= kThreads * kTbPer;
   float f[kTbPer];
   // each(i, score) over this thread's scores, kTbPer loads in flight at a time
   const auto each = [&](bool load, auto use) {
     for (int base = 0; base < n_valid; base += kThreads * kTbPer) {
-      if (load) {
+      if (load || !fits) {
 #pragma unroll
         for (int q = 0; q < kTbPer; ++q) f[q] = row[min(base + q * kThreads + tid, n_valid - 1)];
       }
@@ -225,7 +226,6 @@ __device__ __forceinline__ void topk_row_buckets(TopkBucketSmem<kThreads>& sm, c
       for (int q = 0; q < kTbPer; ++q) {
         if (base + q * kThreads + tid < n_valid) use(base + q * kThreads + tid, f[q]);
       }
-      if (kRegs) break;
     }
   };
   float lo = inf, hi = -inf;
@@ -257,7 +257,7 @@ __device__ __forceinline__ void topk_row_buckets(TopkBucketSmem<kThreads>& sm, c
     const int b = static_cast<int>(x);
     return __builtin_fabsf(v) < inf ? b : (v == -inf ? 0 : kTbBuckets - 1);
   };
-  each(!kRegs, [&](int, float v) { atomicAdd(&sm.u.b.cursor[bucket_of(v)], 1); });
+  each(false, [&](int, float v) { atomicAdd(&sm.u.b.cursor[bucket_of(v)], 1); });
   __syncthreads();
   {
     constexpr int per = kTbBuckets / kThreads;
@@ -289,7 +289,7 @@ __device__ __forceinline__ void topk_row_buckets(TopkBucketSmem<kThreads>& sm, c
     topk_row_emit<kThreads>(sm.u.full, row, n_cols, n_valid, sel, emit);  // its ranks past sel are written
     return;
   }
-  each(!kRegs, [&](int i, float v) {
+  each(false, [&](int i, float v) {
     const int b = bucket_of(v);
     if (sm.u.b.cursor[b] < total) {  // the threshold bucket or above (their slots end at total)
       const int slot = atomicAdd(&sm.u.b.cursor[b], 1);

@@ -48,16 +48,15 @@ __device__ __forceinline__ void topk_row_dims(const TopkArgs& a, int r, int& n_c
   }
 }
 
-// One workgroup per row (topk_row_buckets); kRegs: no row has more than
-// kThreads * kTbPer columns.
-template <int kThreads, bool kRegs>
+// One workgroup per row (topk_row_buckets).
+template <int kThreads>
 __global__ __launch_bounds__(kThreads) void k_topk_rows(TopkArgs a) {
   extern __shared__ char lds[];
   const int r = blockIdx.x;
   int n_cols, n_valid;
   topk_row_dims(a, r, n_cols, n_valid);
   const int64_t at = r * a.out_stride;
-  topk_row_buckets<kThreads, kRegs>(*reinterpret_cast<TopkBucketSmem<kThreads>*>(lds), a.scores + r * a.stride, n_cols,
+  topk_row_buckets<kThreads>(*reinterpret_cast<TopkBucketSmem<kThreads>*>(lds), a.scores + r * a.stride, n_cols,
                                     n_valid, a.k, [&](int j, int v) {
                                       if (a.out64) {
                                         a.out64[at + j] = v;
@@ -203,25 +202,23 @@ __global__ __launch_bounds__(kGatherThreads) void k_topk_gather(TopkGatherArgs a
 
 using namespace skv;
 
-template <int kThreads, bool kRegs>
+template <int kThreads>
 static void launch_topk_rows_as(const TopkArgs& a, int64_t rows, hipStream_t s) {
-  hipLaunchKernelGGL((k_topk_rows<kThreads, kRegs>), dim3(static_cast<unsigned>(rows)), dim3(kThreads),
+  hipLaunchKernelGGL(k_topk_rows<kThreads>, dim3(static_cast<unsigned>(rows)), dim3(kThreads),
                      topk_bucket_lds<kThreads>(a.k), s, a);
 }
 
-// Bounds every row's columns.
+// A row's columns as the host knows them: at least the most a row has, unless rows
+// overlap (a stride below it).
 static int64_t topk_cols(const TopkArgs& a) { return (a.lens || a.n_cols) ? a.stride : a.n_cols_uni; }
 
 static void launch_topk_rows(const TopkArgs& a, int64_t rows, hipStream_t s) {
-  const int64_t cols = topk_cols(a);
   // 256 threads, 16 scores each, where the rows fill the device that way
   // (2,048 rows of 4,096: 7 on a CU at once); one row alone ends sooner with 1,024
-  if (rows >= kTopkManyRows && cols <= 256 * kTbPer) {
-    launch_topk_rows_as<256, true>(a, rows, s);
-  } else if (cols <= kTopkThreads * kTbPer) {
-    launch_topk_rows_as<kTopkThreads, true>(a, rows, s);
+  if (rows >= kTopkManyRows && topk_cols(a) <= 256 * kTbPer) {
+    launch_topk_rows_as<256>(a, rows, s);
   } else {
-    launch_topk_rows_as<kTopkThreads, false>(a, rows, s);
+    launch_topk_rows_as<kTopkThreads>(a, rows, s);
   }
 }
 
