@@ -6,6 +6,8 @@
 // any scores and is the fallback of the faster selections below.
 #pragma once
 
+#include <type_traits>
+
 #include "skv_common.h"
 
 namespace skv {
@@ -163,47 +165,52 @@ __device__ __forceinline__ void topk_row(TopkSmemT<kThreads>& sm, const float* r
 //             positive factor and truncation are).  +inf and NaN go to the top
 //             bucket, -inf to bucket 0.
 //   count   : LDS histogram; its sums from the top give every bucket's first
-//             position and the bucket that holds position sel - 1.
+//             position and the bucket that holds the last pick.  The lowest bucket,
+//             where masks, zeros and all but the outliers heap up, is what remains.
 //   scatter : keys of that bucket and above go to their bucket's slots as
 //             64-bit order keys (key << 32 | ~index).
 //   order   : a candidate's position is its bucket's first plus the candidates
 //             of its bucket above it: a few, where the scores spread.
-// The radix select (topk_row_emit) makes four passes of histograms over the row
-// and ranks every winner against every other; it takes the rows whose buckets
-// hold more than kTbMaxBucket candidates, or more than the LDS does (scores
-// that are nearly all equal or hold an outlier far beyond the rest).
-// Latency-bound: 512 picks of 4,096 scores, 2,048 rows 24 us (391 by the radix
-// select, whose 150 KB of LDS kept one row on a CU), one row 9.9 us (48);
-// of 16,384 scores, 500 rows 17.7 us (122).
+// Where a bucket holds too many (an outlier far beyond the rest, masks of the
+// type's lowest value, ties) the picks above it are written and the same is done
+// among its scores alone: linear between their own ends once more, then by the
+// order key's bits, and for one score that repeats by index; each level takes at
+// least 11 bits off what is left.
+// Latency-bound: 512 picks of 4,096 scores, 2,048 rows 25.8 us (391 by the radix
+// select, whose 150 KB of LDS kept one row on a CU), one row 10.6 us (50); of 16,384
+// scores, 500 rows 20 us (126).  Skewed, by the radix select after a first level /
+// by levels / by the radix select alone: one outlier of 10^6 in 4,096, one row 58 /
+// 15 / 51 us, 2,048 rows 224 / 44 / 392; masks of the lowest float 58 / 16 / 51 and
+// 226 / 54 / 397; zeros for most, of which some are picked, 72 / 20 / 66 and 329 /
+// 62 / 530; one score throughout 83 / 14 / 76 and 363 / 38 / 597.
 // ---------------------------------------------------------------------------
 constexpr int kTbBuckets = 2048;
+constexpr int kTbBits = 11;
 constexpr int kTbPer = 16;         // scores per thread held in registers
-constexpr int kTbMaxBucket = 512;  // candidates of one bucket
-constexpr int kTbSlack = 512;      // LDS candidates beyond k
+constexpr int kTbMaxBucket = 256;  // candidates of one bucket that are compared with one another
 
 template <int kThreads>
 struct TopkBucketSmem {
   int scan_lds[17];
-  int threshold[2];  // candidates at and above the threshold bucket, the fullest of those buckets
-  float lo[kThreads / kWave], hi[kThreads / kWave];
-  union {
-    TopkSmemT<kThreads> full;
-    struct {
-      int cursor[kTbBuckets];
-      uint64_t cand[1];  // k + kTbSlack of them
-    } b;
-  } u;
+  int anchor, threshold, above, count;  // of a level: see there
+  uint32_t lo[kThreads / kWave], hi[kThreads / kWave];
+  int cursor[kTbBuckets];
+  uint64_t cand[1];  // k + kTbMaxBucket of them
 };
 
 // LDS bytes of topk_row_buckets for k picks.
 template <int kThreads>
 constexpr size_t topk_bucket_lds(int k) {
-  const size_t need = offsetof(TopkBucketSmem<kThreads>, u.b.cand) + sizeof(uint64_t) * (k + kTbSlack);
-  return need > sizeof(TopkBucketSmem<kThreads>) ? need : sizeof(TopkBucketSmem<kThreads>);
+  return offsetof(TopkBucketSmem<kThreads>, cand) + sizeof(uint64_t) * (k + kTbMaxBucket);
 }
 
-// emit(j, v) as topk_row_emit calls it.
-template <int kThreads, class Emit>
+// The score of an order key that is not NaN's.
+__device__ __forceinline__ float key_score(uint32_t key) {
+  return __uint_as_float((key & 0x80000000u) ? key & 0x7fffffffu : ~key);
+}
+
+// emit(j, v) as topk_row_emit calls it.  kFits: at most kThreads * kTbPer valid scores.
+template <int kThreads, bool kFits, class Emit>
 __device__ __forceinline__ void topk_row_buckets(TopkBucketSmem<kThreads>& sm, const float* row, int n_cols, int n_valid,
                                                  int k, Emit emit) {
   const int tid = threadIdx.x;
@@ -213,102 +220,216 @@ __device__ __forceinline__ void topk_row_buckets(TopkBucketSmem<kThreads>& sm, c
   for (int j = sel + tid; j < k; j += kThreads) emit(j, -1);
   if (sel == 0) return;
   const float inf = __builtin_huge_valf();
-  const bool fits = n_valid <= kThreads * kTbPer;
   float f[kTbPer];
-  // each(i, score) over this thread's scores, kTbPer loads in flight at a time
+  // each(i, score, in the row) for this thread's places, kTbPer loads in flight at a
+  // time; whole waves call it
   const auto each = [&](bool load, auto use) {
     for (int base = 0; base < n_valid; base += kThreads * kTbPer) {
-      if (load || !fits) {
+      if (load || !kFits) {
 #pragma unroll
         for (int q = 0; q < kTbPer; ++q) f[q] = row[min(base + q * kThreads + tid, n_valid - 1)];
       }
 #pragma unroll
       for (int q = 0; q < kTbPer; ++q) {
-        if (base + q * kThreads + tid < n_valid) use(base + q * kThreads + tid, f[q]);
+        const int i = base + q * kThreads + tid;
+        use(i, f[q], i < n_valid);
+      }
+      if (kFits) break;
+    }
+  };
+  // the same with the scores read again: levels after the first, whose registers
+  // would cost the first a workgroup per CU
+  const auto each_again = [&](auto use) {
+    constexpr int kPer = 4;
+#pragma unroll 1
+    for (int base = 0; base < n_valid; base += kThreads * kPer) {
+      float g[kPer];
+#pragma unroll
+      for (int q = 0; q < kPer; ++q) g[q] = row[min(base + q * kThreads + tid, n_valid - 1)];
+#pragma unroll
+      for (int q = 0; q < kPer; ++q) {
+        const int i = base + q * kThreads + tid;
+        use(i, g[q], i < n_valid);
       }
     }
   };
-  float lo = inf, hi = -inf;
-  each(true, [&](int, float v) {
-    const bool fin = __builtin_fabsf(v) < inf;
-    lo = fin ? fminf(lo, v) : lo;
-    hi = fin ? fmaxf(hi, v) : hi;
-  });
-  for (int b = tid; b < kTbBuckets; b += kThreads) sm.u.b.cursor[b] = 0;
-  if (tid < 2) sm.threshold[tid] = 0;
+  // the workgroup's smallest lo and largest hi; clears the histogram on the way
+  const auto reduce = [&](uint32_t& lo, uint32_t& hi) {
+    for (int b = tid; b < kTbBuckets; b += kThreads) sm.cursor[b] = 0;
+    if (tid == 0) sm.anchor = -1;
 #pragma unroll
-  for (int d = 1; d < kWave; d <<= 1) {
-    lo = fminf(lo, __shfl_xor(lo, d));
-    hi = fmaxf(hi, __shfl_xor(hi, d));
-  }
-  if (tid % kWave == 0) {
-    sm.lo[tid / kWave] = lo;
-    sm.hi[tid / kWave] = hi;
-  }
-  __syncthreads();
+    for (int d = 1; d < kWave; d <<= 1) {
+      lo = min(lo, static_cast<uint32_t>(__shfl_xor(static_cast<int>(lo), d)));
+      hi = max(hi, static_cast<uint32_t>(__shfl_xor(static_cast<int>(hi), d)));
+    }
+    if (tid % kWave == 0) {
+      sm.lo[tid / kWave] = lo;
+      sm.hi[tid / kWave] = hi;
+    }
+    __syncthreads();
 #pragma unroll
-  for (int w = 0; w < kThreads / kWave; ++w) {
-    lo = fminf(lo, sm.lo[w]);
-    hi = fmaxf(hi, sm.hi[w]);
-  }
-  const float scale = hi > lo ? static_cast<float>(kTbBuckets) / (hi - lo) : 0.f;  // 0 too where the range overflows
-  const auto bucket_of = [&](float v) -> int {
+    for (int w = 0; w < kThreads / kWave; ++w) {
+      lo = min(lo, sm.lo[w]);
+      hi = max(hi, sm.hi[w]);
+    }
+    lo = __builtin_amdgcn_readfirstlane(lo);
+    hi = __builtin_amdgcn_readfirstlane(hi);
+  };
+  // A level's scores: keys in [k_lo, k_hi], n_set of them, of which the `want` best
+  // take positions from `first` on.
+  uint32_t k_lo, k_hi;
+  int n_set = n_valid, want = sel, first = 0;
+  // One level over the map bucket(score, index), -1 for scores that are not the
+  // level's.  kFirst: all are.  True when the picks are written; otherwise the
+  // level's last full bucket is in `low`, k_lo..k_hi are its keys, n_set, want and
+  // first what is left, and the histogram is clear.
+  int low;
+  const auto run = [&](auto bucket, auto is_first) -> bool {
+    constexpr bool kFirst = decltype(is_first)::value;
+    const auto scores = [&](auto use) {
+      if constexpr (kFirst) {
+        each(false, use);
+      } else {
+        each_again(use);
+      }
+    };
+    scores([&](int i, float v, bool live) {
+      const int b = live ? bucket(v, i) : 0;
+      if constexpr (kFirst) {
+        if (b > 0) atomicAdd(&sm.cursor[b], 1);
+      } else {
+        const int b0 = __builtin_amdgcn_readfirstlane(b);
+        const int same = __popcll(__ballot(b == b0));
+        if (b > 0 && (b != b0 || tid % kWave == 0)) atomicAdd(&sm.cursor[b], b == b0 ? same : 1);
+      }
+    });
+    __syncthreads();
+    {
+      constexpr int per = kTbBuckets / kThreads;
+      const int b0 = kTbBuckets - 1 - tid * per;  // this thread's buckets: b0, b0 - 1, ...
+      int v[per], sum = 0;
+#pragma unroll
+      for (int q = 0; q < per; ++q) {
+        v[q] = sm.cursor[b0 - q];
+        sum += v[q];
+      }
+      int tot;
+      int ex = block_exclusive_scan(sum, sm.scan_lds, &tot);  // scores in higher buckets
+#pragma unroll
+      for (int q = 0; q < per; ++q) {
+        if (b0 - q == 0) v[q] = n_set - ex;
+        sm.cursor[b0 - q] = ex;
+        if (ex < want) {
+          if (want <= ex + v[q]) {
+            sm.threshold = b0 - q;
+            sm.above = ex;
+            sm.count = v[q];
+          } else if (kFirst && v[q] > kTbMaxBucket) {
+            atomicMax(&sm.anchor, b0 - q);
+          }
+        }
+        ex += v[q];
+      }
+    }
+    __syncthreads();
+    // The bucket of the last pick is `low`; the next level takes buckets [low, high]:
+    // that one, after the first level from the highest that is too full on.
+    low = __builtin_amdgcn_readfirstlane(sm.threshold);
+    const int count = __builtin_amdgcn_readfirstlane(sm.count), above = __builtin_amdgcn_readfirstlane(sm.above);
+    const int high = kFirst ? max(low, __builtin_amdgcn_readfirstlane(sm.anchor)) : low;
+    const bool last = high == low && count <= kTbMaxBucket;
+    const int from = last ? low : high + 1;  // buckets whose picks are written now
+    const int total = last ? above + count : high == low ? above : __builtin_amdgcn_readfirstlane(sm.cursor[high]);
+    if (total > 0) {
+      if (kFirst && high > low) __syncthreads();  // a cursor has been read
+      scores([&](int i, float v, bool live) {
+        const int b = live ? bucket(v, i) : -1;
+        if (b < from) return;
+        sm.cand[atomicAdd(&sm.cursor[b], 1)] = (static_cast<uint64_t>(score_key(v)) << 32) | static_cast<uint32_t>(~i);
+      });
+      __syncthreads();
+      for (int c = tid; c < total; c += kThreads) {
+        const uint64_t key = sm.cand[c];
+        const uint32_t hi_key = static_cast<uint32_t>(key >> 32);
+        const int i = static_cast<int>(~static_cast<uint32_t>(key));
+        const int b = bucket(key_score(hi_key), i);
+        const int begin = b == kTbBuckets - 1 ? 0 : sm.cursor[b + 1];  // the next bucket's end
+        if (begin >= want) continue;
+        const int end = sm.cursor[b];
+        int rank = 0, j = begin;
+        for (; j + 8 <= end; j += 8) {
+#pragma unroll
+          for (int u = 0; u < 8; ++u) rank += sm.cand[j + u] > key;
+        }
+        for (; j < end; ++j) rank += sm.cand[j] > key;
+        if (begin + rank < want) emit(first + begin + rank, key_finite(hi_key) ? i : -1);
+      }
+    }
+    if (last) return true;
+    k_lo = ~0u;
+    k_hi = 0u;
+    each_again([&](int i, float v, bool live) {
+      const int b = live ? bucket(v, i) : -1;
+      if (b < low || b > high) return;
+      k_lo = min(k_lo, score_key(v));
+      k_hi = max(k_hi, score_key(v));
+    });
+    __syncthreads();  // the cursors have been read
+    reduce(k_lo, k_hi);
+    n_set = above + count - total;
+    want -= total;
+    first += total;
+    return false;
+  };
+  // linear in the scores from lo to hi: not finite ones to the ends
+  float lo, scale;
+  const auto by_score = [&](float v, int) -> int {
     const float x = fminf(fmaxf((v - lo) * scale, 0.f), static_cast<float>(kTbBuckets - 1));
     const int b = static_cast<int>(x);
     return __builtin_fabsf(v) < inf ? b : (v == -inf ? 0 : kTbBuckets - 1);
   };
-  each(false, [&](int, float v) { atomicAdd(&sm.u.b.cursor[bucket_of(v)], 1); });
-  __syncthreads();
-  {
-    constexpr int per = kTbBuckets / kThreads;
-    const int top = kTbBuckets - 1 - tid * per;  // this thread's buckets: top, top - 1, ...
-    int v[per], sum = 0;
-#pragma unroll
-    for (int q = 0; q < per; ++q) {
-      v[q] = sm.u.b.cursor[top - q];
-      sum += v[q];
-    }
-    int tot;
-    int ex = block_exclusive_scan(sum, sm.scan_lds, &tot);  // scores in higher buckets
-    int fullest = 0;
-#pragma unroll
-    for (int q = 0; q < per; ++q) {
-      sm.u.b.cursor[top - q] = ex;
-      if (ex < sel) {
-        fullest = max(fullest, v[q]);
-        if (sel <= ex + v[q]) sm.threshold[0] = ex + v[q];
-      }
-      ex += v[q];
-    }
-    if (fullest > kTbMaxBucket) atomicMax(&sm.threshold[1], fullest);
-  }
-  __syncthreads();
-  const int total = sm.threshold[0];
-  if (__builtin_expect(total > k + kTbSlack || sm.threshold[1] > kTbMaxBucket, 0)) {  // uniform
-    __syncthreads();
-    topk_row_emit<kThreads>(sm.u.full, row, n_cols, n_valid, sel, emit);  // its ranks past sel are written
-    return;
-  }
-  each(false, [&](int i, float v) {
-    const int b = bucket_of(v);
-    if (sm.u.b.cursor[b] < total) {  // the threshold bucket or above (their slots end at total)
-      const int slot = atomicAdd(&sm.u.b.cursor[b], 1);
-      sm.u.b.cand[slot] = (static_cast<uint64_t>(score_key(v)) << 32) | static_cast<uint32_t>(~i);
-    }
+  lo = inf;
+  float hi = -inf;
+  each(true, [&](int, float v, bool) {
+    const bool fin = __builtin_fabsf(v) < inf;
+    lo = fin ? fminf(lo, v) : lo;
+    hi = fin ? fmaxf(hi, v) : hi;
   });
-  __syncthreads();
-  for (int c = tid; c < total; c += kThreads) {
-    const uint64_t key = sm.u.b.cand[c];
-    const uint32_t hi_key = static_cast<uint32_t>(key >> 32);
-    // the score's bits (every NaN is in the top bucket)
-    const uint32_t bits = (hi_key & 0x80000000u) ? hi_key & 0x7fffffffu : ~hi_key;
-    const int b = bucket_of(hi_key == kKeyNaN ? inf : __uint_as_float(bits));
-    const int first = b == kTbBuckets - 1 ? 0 : sm.u.b.cursor[b + 1];  // the next bucket's end
-    if (first >= sel) continue;
-    const int end = sm.u.b.cursor[b];
-    int rank = 0;
-    for (int j = first; j < end; ++j) rank += sm.u.b.cand[j] > key;
-    if (first + rank < sel) emit(first + rank, key_finite(hi_key) ? static_cast<int>(~static_cast<uint32_t>(key)) : -1);
+  k_lo = score_key(lo);
+  k_hi = score_key(hi);
+  reduce(k_lo, k_hi);
+  lo = k_lo <= k_hi ? key_score(k_lo) : 0.f;
+  scale = k_lo < k_hi ? static_cast<float>(kTbBuckets) / (key_score(k_hi) - lo) : 0.f;  // 0 too where the range overflows
+  if (run(by_score, std::true_type{})) return;
+  {
+    hi = key_score(k_hi);
+    lo = key_score(k_lo);
+    scale = static_cast<float>(kTbBuckets) / (hi - lo);
+    if (scale > 0.f && scale < inf) {  // two finite scores
+      if (run([&](float v, int i) { return v >= lo && v <= hi ? by_score(v, i) : -1; }, std::false_type{})) return;
+    }
+  }
+  const auto bits = [](uint32_t range) { return range >> kTbBits ? 32 - kTbBits - __builtin_clz(range) : 0; };
+  while (k_lo != k_hi) {
+    const uint32_t base = k_lo, range = k_hi - k_lo;
+    const int shift = bits(range);
+    const auto by_key = [&](float v, int) {
+      const uint32_t d = score_key(v) - base;
+      return d <= range ? static_cast<int>(d >> shift) : -1;
+    };
+    if (run(by_key, std::false_type{})) return;
+  }
+  uint32_t i_lo = 0, range = n_valid - 1;
+  for (;;) {
+    const uint32_t base = k_lo;
+    const int shift = bits(range);
+    const auto by_index = [&](float v, int i) {
+      const uint32_t d = i - i_lo;
+      return score_key(v) == base && d <= range ? kTbBuckets - 1 - static_cast<int>(d >> shift) : -1;
+    };
+    if (run(by_index, std::false_type{})) return;
+    i_lo += static_cast<uint32_t>(kTbBuckets - 1 - low) << shift;
+    range = (1u << shift) - 1;  // none past the row's end is live
   }
 }
 

@@ -48,22 +48,30 @@ __device__ __forceinline__ void topk_row_dims(const TopkArgs& a, int r, int& n_c
   }
 }
 
-// One workgroup per row (topk_row_buckets).
+// One workgroup per row (topk_row_buckets).  The bounds keep two workgroups of 1,024
+// threads, or seven of 256, on a CU: the levels after the first, rarely reached,
+// would take more registers (500 rows of 16,384: 25 us, not 20).
 template <int kThreads>
-__global__ __launch_bounds__(kThreads) void k_topk_rows(TopkArgs a) {
+__global__ __launch_bounds__(kThreads, kThreads == kTopkThreads ? 8 : 7) void k_topk_rows(TopkArgs a) {
   extern __shared__ char lds[];
   const int r = blockIdx.x;
   int n_cols, n_valid;
   topk_row_dims(a, r, n_cols, n_valid);
   const int64_t at = r * a.out_stride;
-  topk_row_buckets<kThreads>(*reinterpret_cast<TopkBucketSmem<kThreads>*>(lds), a.scores + r * a.stride, n_cols,
-                                    n_valid, a.k, [&](int j, int v) {
-                                      if (a.out64) {
-                                        a.out64[at + j] = v;
-                                      } else {
-                                        a.out[at + j] = v;
-                                      }
-                                    });
+  auto& sm = *reinterpret_cast<TopkBucketSmem<kThreads>*>(lds);
+  const auto emit = [&](int j, int v) {
+    if (a.out64) {
+      a.out64[at + j] = v;
+    } else {
+      a.out[at + j] = v;
+    }
+  };
+  // a row's own count decides: overlapping rows have more columns than their stride
+  if (min(n_valid, n_cols) <= kThreads * kTbPer) {
+    topk_row_buckets<kThreads, true>(sm, a.scores + r * a.stride, n_cols, n_valid, a.k, emit);
+  } else {
+    topk_row_buckets<kThreads, false>(sm, a.scores + r * a.stride, n_cols, n_valid, a.k, emit);
+  }
 }
 
 // Multi-workgroup form: hist and filter over grid (chunks, rows), final over
@@ -233,10 +241,12 @@ static int launch_topk(const TopkArgs& a, int64_t rows, int32_t* workspace, void
   if (rows == 0 || a.k == 0) return SKV_OK;
   hipStream_t s = static_cast<hipStream_t>(stream);
   // A row of up to 16,384 columns stays in one workgroup's registers, which
-  // beats the three launches whatever the row count (512 of 16,384: 1 row 11.6
-  // against 18.0 us, 500 rows 17.7 against 47.7); longer rows are read three
-  // times by one workgroup (1,024 of 65,536: 31.0 against 27.5 us, of 262,144:
-  // 99 against 31) and take the launches where the caller gives a workspace.
+  // beats the three launches whatever the row count (512 of 16,384: 1 row 12.7
+  // against 19.2 us, 500 rows 19 against 48) but for a few rows whose scores take a
+  // second level (an outlier of 10^6 24 against 19; masks of the lowest float 29
+  // against 19); longer rows are read three times by one workgroup (1,024 of 65,536:
+  // 33 against 30 us, of 262,144: 99 against 31) and take the launches where the
+  // caller gives a workspace.
   if (!workspace || topk_cols(a) <= kTopkThreads * kTbPer) {
     launch_topk_rows(a, rows, s);
     return check_launch(what);
