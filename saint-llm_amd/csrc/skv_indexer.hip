@@ -71,7 +71,7 @@ __global__ __launch_bounds__(kIdxThreads, 2) void k_indexer_scores(IndexerArgs a
 // before; a large bf16 product of the library runs at 1.27).  Two tokens per
 // wave would halve the key reads but spill.
 // ---------------------------------------------------------------------------
-constexpr int kIrMinTokens = 6;  // fewer query tokens per sequence: k_indexer_scores (see the launch)
+constexpr int kIrMinTokens = 6;  // fewer query tokens per sequence: k_indexer_scores, as for few tiles (see the launch)
 constexpr int kIrThreads = 512;
 constexpr int kIrTokens = kIrThreads / kWave;  // query tokens per workgroup, one per wave
 constexpr int kIrTile = 128;                   // entries per LDS tile
@@ -258,9 +258,16 @@ void launch_indexer_rows(const IndexerArgs& a, int64_t batch, hipStream_t s) {
 template <bool kChunk>
 void launch_indexer(const IndexerArgs& a, int64_t batch, hipStream_t s) {
   // The line: 16 x 16,384 entries and 64 heads take k_indexer_scores 42 us for 4
-  // tokens and 10.5 us for each more, k_indexer_scores_rows 53 us for 4 to 8.
-  if (a.t_per_seq >= kIrMinTokens) {
-    const int hb = a.n_heads <= 16 ? 1 : a.n_heads <= 32 ? 2 : 4, ks = a.c <= 32 ? 1 : a.c <= 64 ? 2 : 4;
+  // tokens and 10.5 us for each more, k_indexer_scores_rows 53 us for 4 to 8.  While
+  // the tiles of k_indexer_scores are too few to fill the device, the long start of
+  // the other's workgroups counts for more, the larger the query the longer (scores /
+  // rows; 64 heads x 128: 1 tile a CU 8.4 / 12.4 us, 2 12.6 / 12.7, 3 18.4 / 14.1;
+  // 64 x 64: 1 7.1 / 8.6, 2 10.2 / 8.8; 32 x 128: an eighth 6.7 / 7.9, three eighths
+  // 8.0 / 8.0; smaller ones 6.5 / 4.2-6.3 from the first tile on).
+  const int hb = a.n_heads <= 16 ? 1 : a.n_heads <= 32 ? 2 : 4, ks = a.c <= 32 ? 1 : a.c <= 64 ? 2 : 4;
+  const int quarters = hb * ks == 16 ? 10 : hb == 4 && ks == 2 ? 6 : hb * ks == 8 ? 1 : 0;  // tiles per four CUs
+  const int64_t tiles = batch * a.t_per_seq * ceil_div(a.max_entries, kIdxTile);
+  if (a.t_per_seq >= kIrMinTokens && 4 * tiles >= quarters * static_cast<int64_t>(device_cus())) {
     switch (hb * 8 + ks) {
       case 9: launch_indexer_rows<1, 1, kChunk>(a, batch, s); break;
       case 10: launch_indexer_rows<1, 2, kChunk>(a, batch, s); break;

@@ -39,3 +39,26 @@ def test_indexer_scores_rows(dev, t, h, c, n_max) -> None:
         ops.indexer_scores(q[:, i:i + 1].contiguous(), w[:, i:i + 1].contiguous(), pool, table, n_ent, one,
                            max_entries=n_max)
         assert torch.equal(got[:, i].view(torch.int32), one[:, 0].view(torch.int32)), i
+
+
+@pytest.mark.parametrize("batch,t,h,c,n_max", [(120, 6, 64, 128, 129), (100, 7, 64, 120, 1), (8, 33, 33, 64, 1000),
+                                               (64, 9, 50, 40, 513), (20, 6, 32, 128, 127), (12, 17, 17, 72, 300)])
+def test_large_queries_of_many_sequences(dev, batch, t, h, c, n_max) -> None:
+    """Queries that take the rows' kernel only where its tiles fill the device, against a token at a time."""
+    from saint_kv import ops
+
+    g = torch.Generator().manual_seed(batch + h)
+    n_ent = torch.randint(0, n_max + 1, (batch,), generator=g, dtype=torch.int32)
+    n_ent[0], n_ent[-1] = n_max, 0
+    n_ent = n_ent.to(dev)
+    pages = -(-n_max // 16)
+    table = torch.randperm(batch * pages, generator=g).view(batch, pages).to(torch.int32).to(dev)
+    pool = torch.randn(batch * pages, 16, c, generator=g).to(torch.bfloat16).to(dev)
+    q = torch.randn(batch, t, h, c, generator=g).to(torch.bfloat16).to(dev)
+    w = torch.randn(batch, t, h, generator=g).to(dev)
+    got = torch.full((batch, t, n_max), 7.0, device=dev)
+    ops.indexer_scores(q, w, pool, table, n_ent, got)
+    for i in range(t):
+        one = torch.full((batch, 1, n_max), 7.0, device=dev)
+        ops.indexer_scores(q[:, i:i + 1].contiguous(), w[:, i:i + 1].contiguous(), pool, table, n_ent, one)
+        assert torch.equal(got[:, i].view(torch.int32), one[:, 0].view(torch.int32)), i
