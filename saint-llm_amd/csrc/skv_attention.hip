@@ -874,6 +874,44 @@ struct AttnPlan {
   int64_t ws_bytes;
 };
 
+// Whether `items` (query row, 64 heads) take a workgroup each (k_attn_rows) rather than
+// units and a merge.  From two CUs an item on the split has an item's two branches
+// in a unit each, and one workgroup for both of them is faster by what the merge and
+// the units' barriers cost, the more so the more of its work is compressed keys.
+// Against it count: score waves without heads (of every 64, 16 a wave), fp8
+// entries (dequantized by the waves that compute), dims far below the 512 or 576
+// that its registers are made for, a window alone, and a last round of workgroups
+// that is nearly empty, which the split's shorter units fill better.  Time over the
+// split's, a window of 128, 256 CUs (compressed keys: 64 picks to 1,000 entries):
+//   items            128        130-256    260-384     512        1,024
+//   64 x 576         0.74-0.91  0.49-0.62  0.59-0.76   0.49-0.60  0.49-0.63
+//   64 x 576 fp8     0.94-1.09  0.58-0.74  0.73-0.91   0.63-0.73  0.63-0.72
+//   16 x 576         0.98-1.24  0.54-0.80  0.71-0.99   0.56-0.77  0.64-0.79
+//   16 x 576 fp8     1.09-1.47  0.63-0.96  0.88-1.23   0.71-0.93  0.72-1.01
+//   16 x 160-256     1.2-1.5    0.5-0.99   0.67-1.28   0.6-1.02   0.5-1.01
+//   8-64 x 128       0.76-1.13  0.56-0.98  0.48-0.80   0.39-0.73  0.40-0.72
+//   window alone: 64 x 576 0.75-0.80, 0.50-0.67, 0.66-0.88, 0.56, 0.63; 16 x 576
+//   1.10-1.25, 0.70-0.84, 0.97-1.03, 0.89, 0.92; 16 x 256 1.2-1.4, 0.9-1.2, 1.2-1.35,
+//   1.15, 1.23; 64 x 256 1.1, 0.75-0.85, 1.03-1.15, 0.95, 0.98
+// Wider windows' scores do not fit its LDS.
+bool attn_by_rows(const skv_attention_desc* d, int64_t items) {
+  const int64_t cus = device_cus(), groups = ceil_div(d->n_heads, kAtHeads);
+  if (d->splits > 0 || d->window > kRowsMaxWindow || 2 * items < cus) return false;
+  const bool fp8 = d->kind != SKV_LAYER_SWA && d->format == SKV_FMT_FP8;
+  const int64_t dim = d->head_dim;
+  // the split's units are one round of workgroups
+  if (2 * items == cus) return d->n_heads % kAtHeads == 0 && !fp8 && (dim <= 128 || dim > 512);
+  if (dim <= 128) return true;
+  const bool full = d->n_heads > 48 * groups;  // all four score waves have heads
+  if (d->kind == SKV_LAYER_SWA) {
+    return items <= cus ? dim >= 384 || d->n_heads >= 32 * groups
+                        : full ? dim >= 384 : d->n_heads == 48 * groups && dim >= 512;
+  }
+  if (items <= cus || full) return true;
+  const int64_t places = ceil_div(items, cus) * cus;  // of its rounds
+  return fp8 || dim < 512 ? 8 * items >= 7 * places : 10 * items >= 7 * places;
+}
+
 int attn_plan(const skv_attention_desc* d, AttnPlan& p) {
   const char* what = "skv_decode_attention";
   if (!d) return set_error(SKV_EINVAL, "%s: NULL descriptor", what);
@@ -965,12 +1003,7 @@ int attn_plan(const skv_attention_desc* d, AttnPlan& p) {
   p.n_wu = static_cast<int>(n_wu);
   const int64_t units = p.rows * (n_cu + n_wu) * p.n_hg;
   if (units >= (1 << 30)) return set_error(SKV_EINVAL, "%s: too many workgroups", what);
-  // From a row per two CUs on a row is not split further (its two branches fill
-  // the device), and one workgroup for both of them is faster than two units and a
-  // merge (512 picks and a window of 128, 64 heads x 576: 128 rows 58 against 67 us,
-  // 256 rows 60 against 115, 512 rows 114 against 216); wider windows' scores do
-  // not fit its LDS.
-  p.by_rows = d->splits <= 0 && d->window <= kRowsMaxWindow && 2 * p.rows * p.n_hg >= device_cus();
+  p.by_rows = attn_by_rows(d, p.rows * p.n_hg);
   p.ws_bytes = units * kAtHeads * (2 * static_cast<int64_t>(sizeof(float)) + d->head_dim * 2);  // (max, sum) fp32, O bf16
   return SKV_OK;
 }
