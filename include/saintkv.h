@@ -525,9 +525,13 @@ int skv_decode_step_launches(const skv_decode_desc* host_desc);
  * The pool's entries are bf16 or fp8 (dequantized to bf16 as the gathers
  * do).  Two launches: per (sequence, split, 64 heads) partial softmax
  * statistics and outputs into `workspace` (16-byte aligned), then the merge
- * into `out` (fp32).
- * skv_attention_workspace returns the workspace bytes (or -1 on a bad
- * descriptor). */
+ * into `out` (fp32); or, where the query rows fill the device (splits 0,
+ * window <= 128), one launch with a workgroup per row and 64 heads, which
+ * leaves the workspace as it is.
+ * skv_attention_workspace returns the workspace bytes that the call asks for
+ * (or -1 on a bad descriptor): what its units need, of a call in one launch
+ * no more than the calls of fewer rows do, so that a workspace made for the
+ * most rows serves them all. */
 typedef struct skv_attention_desc {
   int32_t kind;             /* SKV_LAYER_SWA / SKV_LAYER_HCA / SKV_LAYER_CSA */
   int32_t format;           /* SKV_FMT_* of the pool's entries */

@@ -868,11 +868,16 @@ namespace skv {
 
 struct AttnPlan {
   int n_cu, n_wu, n_hg, nks;
-  bool by_rows;  // one workgroup per (query row, head group): k_attn_rows, no workspace
+  bool by_rows;  // one workgroup per (query row, head group): k_attn_rows, which leaves the workspace as it is
   int64_t rows;  // query rows: batch x query tokens per sequence
   int64_t nq, ring, win_row;
-  int64_t ws_bytes;
+  int64_t ws_bytes;  // of the units
 };
+
+// A unit's partial output in the workspace: (max, sum) fp32 and O bf16 per head.
+int64_t attn_unit_bytes(const skv_attention_desc* d) {
+  return kAtHeads * (2 * static_cast<int64_t>(sizeof(float)) + d->head_dim * 2);
+}
 
 // Whether `items` (query row, 64 heads) take a workgroup each (k_attn_rows) rather than
 // units and a merge.  From two CUs an item on the split has an item's two branches
@@ -910,6 +915,18 @@ bool attn_by_rows(const skv_attention_desc* d, int64_t items) {
   if (items <= cus || full) return true;
   const int64_t places = ceil_div(items, cus) * cus;  // of its rounds
   return fp8 || dim < 512 ? 8 * items >= 7 * places : 10 * items >= 7 * places;
+}
+
+// Workspace of a call.  By rows it uses none, and takes what the largest call of fewer
+// rows of the same shape that is split needs, so that a workspace made for the most
+// rows serves fewer: units are at most half more than CUs below the rule's first line,
+// and two an item in rounds that it leaves to the split (up to 2.1 items a CU, of fp8
+// entries and small dims 6.125).  1,000 rows of 64 heads x 576: 28 MB, split 148.
+int64_t attn_workspace(const skv_attention_desc* d, const AttnPlan& p) {
+  if (!p.by_rows) return p.ws_bytes;
+  const bool always = d->kind == SKV_LAYER_SWA || d->head_dim <= 128 || d->n_heads > 48 * ceil_div(d->n_heads, kAtHeads);
+  const int64_t eighths = always ? 12 : d->format == SKV_FMT_FP8 || d->head_dim < 512 ? 98 : 34;  // units per 8 CUs
+  return std::min(p.ws_bytes, ceil_div(eighths * device_cus(), 8) * attn_unit_bytes(d));
 }
 
 int attn_plan(const skv_attention_desc* d, AttnPlan& p) {
@@ -1004,7 +1021,7 @@ int attn_plan(const skv_attention_desc* d, AttnPlan& p) {
   const int64_t units = p.rows * (n_cu + n_wu) * p.n_hg;
   if (units >= (1 << 30)) return set_error(SKV_EINVAL, "%s: too many workgroups", what);
   p.by_rows = attn_by_rows(d, p.rows * p.n_hg);
-  p.ws_bytes = units * kAtHeads * (2 * static_cast<int64_t>(sizeof(float)) + d->head_dim * 2);  // (max, sum) fp32, O bf16
+  p.ws_bytes = units * attn_unit_bytes(d);
   return SKV_OK;
 }
 
@@ -1625,7 +1642,7 @@ extern "C" int64_t skv_attention_desc_size(void) { return static_cast<int64_t>(s
 extern "C" int64_t skv_attention_workspace(const skv_attention_desc* d) {
   AttnPlan p;
   if (attn_plan(d, p) != SKV_OK) return -1;
-  return p.ws_bytes;
+  return attn_workspace(d, p);
 }
 
 extern "C" int skv_decode_attention(const skv_attention_desc* d, void* workspace, int64_t ws_bytes,
@@ -1641,8 +1658,8 @@ extern "C" int skv_decode_attention(const skv_attention_desc* d, void* workspace
       (d->kind == SKV_LAYER_CSA && !d->picks)) {
     return set_error(SKV_EINVAL, "%s: NULL pointer", what);
   }
-  if (!workspace || ws_bytes < p.ws_bytes) {
-    return set_error(SKV_EINVAL, "%s: workspace of %lld bytes needed", what, (long long)p.ws_bytes);
+  if (const int64_t need = attn_workspace(d, p); !workspace || ws_bytes < need) {
+    return set_error(SKV_EINVAL, "%s: workspace of %lld bytes needed", what, (long long)need);
   }
   if (reinterpret_cast<uintptr_t>(workspace) & 15) {
     return set_error(SKV_EINVAL, "%s: workspace must be 16-byte aligned (the merge reads it in vectors)", what);
