@@ -39,9 +39,6 @@ __device__ __forceinline__ void topk_row_dims(const TopkArgs& a, int r, int& n_c
     const int L = max(a.lens[r], 0);
     n_cols = L / a.m;
     n_valid = L > 0 ? (L - 1) / a.m : 0;
-  } else if (a.t_new > 0) {
-    n_cols = a.n_cols_uni;
-    n_valid = (a.offset + r % a.t_new) / a.m;
   } else {
     n_cols = a.n_cols ? a.n_cols[r] : a.n_cols_uni;
     n_valid = a.n_valid[r];
@@ -56,7 +53,12 @@ __global__ __launch_bounds__(kThreads, kThreads == kTopkThreads ? 8 : 7) void k_
   extern __shared__ char lds[];
   const int r = blockIdx.x;
   int n_cols, n_valid;
-  topk_row_dims(a, r, n_cols, n_valid);
+  if (a.t_new > 0) {  // here alone: each of the three launches would wait for one more argument
+    n_cols = a.n_cols_uni;
+    n_valid = (a.offset + r % a.t_new) / a.m;
+  } else {
+    topk_row_dims(a, r, n_cols, n_valid);
+  }
   const int64_t at = r * a.out_stride;
   auto& sm = *reinterpret_cast<TopkBucketSmem<kThreads>*>(lds);
   const auto emit = [&](int j, int v) {
