@@ -84,10 +84,13 @@ class _PagedRows:
         self.pool = torch.zeros(n_pages, block_size, *store_shape, dtype=dtype, device=device)
         self.free_stack = torch.empty(n_pages, dtype=torch.int32, device=device)
         self.free_top = torch.empty(1, dtype=torch.int32, device=device)
-        self.block_table = torch.full((batch, self.max_pages), -1, dtype=torch.int32, device=device)
+        # the block table (unmapped) and reset's release mask (any byte but 0) in one fill
+        words = batch * self.max_pages
+        fill = torch.full((words + -(-batch // 4),), -1, dtype=torch.int32, device=device)
+        self.block_table = fill[:words].view(batch, self.max_pages)
+        self._all = fill[words:].view(torch.uint8)[:batch]
         self.lens = torch.zeros(batch, dtype=torch.int32, device=device)
         self.status = torch.zeros(1, dtype=torch.int32, device=device)
-        self._all: Tensor | None = None  # reset's release mask, made by the first one
         self._out = torch.zeros(batch, max_rows, *store_shape, dtype=dtype, device=device)
         ops.free_stack_init(self.free_stack, self.free_top)
         self.length = 0
@@ -112,8 +115,6 @@ class _PagedRows:
 
     def reset(self) -> None:
         if self.length:
-            if self._all is None:
-                self._all = torch.ones(self.batch, dtype=torch.uint8, device=self.pool.device)
             ops.release(self.free_stack, self.free_top, self.block_table, self.lens, self._all,
                         self.block_size, self.status)
         self.length = 0
