@@ -86,7 +86,7 @@ def indexer_topk(q_indexer: torch.Tensor, head_weights: torch.Tensor, k_indexer_
         out = torch.empty(b, t_new, k_eff, dtype=torch.long, device=dev)
         # an m past every position shows nothing, whatever its value
         return ops.indexer_topk_chunk(q_indexer.to(torch.bfloat16).contiguous(), head_weights.float().contiguous(),
-                                      keys, n_blocks, int(cache_offset), min(int(m), int(total_len) + 1), out)
+                                      keys, n_blocks, int(cache_offset), min(int(m), int(total_len)), out)
     scores = lightning_indexer_scores(q_indexer, k_indexer_comp[:, :n_blocks], head_weights)  # (B, t_new, n)
     # visible entries of the query at position q: s < floor(q / m) (s * m + m - 1 < q)
     q_pos = torch.arange(cache_offset, total_len, device=dev, dtype=torch.int64)

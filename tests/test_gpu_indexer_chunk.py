@@ -46,3 +46,14 @@ def test_picks_equal_the_general_route(b, t_new, h, c, offset, n_blocks, rows, m
     ops.topk_select(scores, torch.tensor(seen, dtype=torch.int32, device=dev), n_blocks, k_eff, want)
     assert got.dtype == torch.int64 and tuple(got.shape) == (b, t_new, k_eff)
     assert torch.equal(got.view(b * t_new, k_eff), want.long())
+
+
+@pytest.mark.parametrize("m,seen", [(2 ** 40, 0), (2 ** 31 - 1, 0), (2 ** 31 - 2, 1)])
+def test_last_position(m, seen) -> None:
+    """The position 2^31 - 2 and blocks about as long: an entry is seen once its block is complete before it."""
+    from saint_kv.indexer import indexer_topk
+
+    dev, last = torch.device("cuda:0"), 2 ** 31 - 2
+    q, k = torch.ones(1, 1, 4, 8, device=dev), torch.ones(1, 3, 8, device=dev)
+    got = indexer_topk(q, torch.ones(1, 1, 4, device=dev), k, cache_offset=last, total_len=last + 1, n_blocks=3, m=m, top_k=2)
+    assert got.tolist() == [[[0, -1] if seen else [-1, -1]]]
