@@ -250,7 +250,8 @@ int skv_compress_append(void* pool, int64_t entry_bytes, int64_t block_size, int
                         int64_t m, int64_t channels, int32_t format, int64_t batch, void* stream);
 
 /* The same for several streams (layers, or a layer's main and indexer stream) of
- * one batch at once: streams whose c/z rows have one type share a launch. */
+ * one batch at once: neighbours whose c/z rows have one type share a launch, up
+ * to 16 of them.  No stream appears twice. */
 typedef struct skv_compress_stream {
   void* pool;
   int64_t entry_bytes, block_size, n_pages;

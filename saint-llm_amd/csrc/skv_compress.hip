@@ -361,7 +361,7 @@ struct CompressStreams {
   int32_t zparts[kCmStreams];  // workgroups over the channels
   int32_t slots[kCmStreams];   // entries of a workgroup at a time
   int32_t channels[kCmStreams];  // of a lane: 8, 2 or 1
-  int32_t n, batch;
+  int32_t n;
 };
 
 template <class Row>
@@ -458,7 +458,6 @@ static int compress_streams(const char* what, const skv_compress_stream* streams
   if (!n_new && n_new_uniform < 0) return set_error(SKV_EINVAL, "%s: n_new_uniform must be >= 0", what);
   if (batch == 0) return SKV_OK;
   CompressStreams cs{};
-  cs.batch = static_cast<int32_t>(batch);
   int64_t blocks = 0;
   for (int64_t i = 0; i < n_streams; ++i) {
     if (streams[i].in_len <= 0) continue;
