@@ -344,8 +344,8 @@ __device__ __forceinline__ void compress_workgroup(CompressSmem& sm, const Compr
 // The streams of one launch, their workgroups one after another: a stream of
 // short blocks or few channels leaves the device partly idle at its end and a small
 // one all along, and each call costs the host more than a small one takes.  Five
-// streams (three layers; 4 prompts of 6,700-8,192 tokens): 112 us in five launches,
-// 73 in one (3.1 TB/s).
+// streams (three layers; 4 prompts of 29,588 tokens in all, 235 MB of c and z rows):
+// 84.5 us, 2.8 TB/s.
 constexpr int kCmStreams = 16;
 // Workgroups of a stream (65,535 sequences of 16 blocks of channels are fewer).  All
 // streams together keep below the 2^32 threads of a launch, past which the runtime

@@ -34,7 +34,7 @@ def _scores(kind: str, rows: int, n: int, rng) -> np.ndarray:
     elif kind == "cauchy":
         s = rng.standard_cauchy((rows, n)).astype(np.float32)
     elif kind == "wide":  # every exponent
-        s = np.ldexp(s, rng.integers(-149, 128, (rows, n))).astype(np.float32)
+        s = np.ldexp(s, rng.integers(-149, 125, (rows, n))).astype(np.float32)
     elif kind == "two":
         s = np.where(s > 0.3, np.float32(1), np.nextafter(np.float32(1), np.float32(2)))
     elif kind == "nan":
