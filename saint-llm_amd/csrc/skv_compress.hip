@@ -356,10 +356,10 @@ static_assert(65535 * (kPoolWave * 8 * kMaxGroups / kCmBlock) <= kCmMaxBlocks &&
 
 struct CompressStreams {
   CompressArgs s[kCmStreams];
-  int32_t first[kCmStreams];  // first workgroup
-  int32_t turns[kCmStreams];  // workgroups over a sequence's blocks
-  int32_t zparts[kCmStreams];  // workgroups over the channels
-  int32_t slots[kCmStreams];   // entries of a workgroup at a time
+  int32_t first[kCmStreams];     // first workgroup
+  int32_t turns[kCmStreams];     // workgroups over a sequence's blocks
+  int32_t zparts[kCmStreams];    // workgroups over the channels
+  int32_t slots[kCmStreams];     // entries of a workgroup at a time
   int32_t channels[kCmStreams];  // of a lane: 8, 2 or 1
   int32_t n;
 };
@@ -470,7 +470,6 @@ static int compress_streams(const char* what, const skv_compress_stream* streams
     }
     if (cs.n == 0) blocks = 0;
     run_f32 = f32;
-    // a call's tokens lie in at most ceil((in_len - 1) / m) + 1 blocks
     // a call's tokens lie in at most ceil((in_len - 1) / m) + 1 blocks
     const int64_t units = ceil_div(a.in_len - 1, a.m) + 1, zblocks = ceil_div(a.channels, kCmBlock);
     const int64_t tokens = std::min<int64_t>(a.m, a.in_len);  // most of an entry
